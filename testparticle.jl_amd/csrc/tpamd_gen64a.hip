@@ -1,6 +1,6 @@
 // tpamd_gen64a.hip -- the generic FP64 kernels for analytic fields (zero, uniform, affine,
 // dipole, E = -u x B of those).
-#include "tpamd_pusher.h"
+#include "tpamd_quad.h"
 
 namespace tpamd {
 
@@ -14,7 +14,7 @@ void launch_generic64_analytic(const LaunchReq& r, int alg, bool special)
         r.p->bnd_flags == 0) {
         const long long threads = 4 * r.p->N;
         const dim3 g((unsigned)((threads + r.b.x - 1) / r.b.x));
-        hipLaunchKernelGGL(k_fixed_quad, g, r.b, 0, r.st, *r.p);
+        hipLaunchKernelGGL((k_fixed_quad<double, quad::Move64>), g, r.b, 0, r.st, *r.p);
         return;
     }
     if (special && !r.batch && !r.adaptive && alg == 0 && r.p->uniform_fields && r.p->rec_w == 6) {
