@@ -1,5 +1,6 @@
 // tpamd_gen64a.hip -- the generic FP64 kernels for analytic fields (zero, uniform, affine,
 // dipole, E = -u x B of those).
+#include "tpamd_dipole.h"
 #include "tpamd_quad.h"
 
 namespace tpamd {
@@ -25,7 +26,7 @@ void launch_generic64_analytic(const LaunchReq& r, int alg, bool special)
     // that pair of fields
     if (special && !r.batch && !r.adaptive && alg == 0 && r.p->rec_w == 6 && r.p->B.kind == kFieldDipole &&
         r.p->E.kind == kFieldZero && !r.p->e_is_uxb) {
-        hipLaunchKernelGGL((k_fixed<DipoleOnly<S64A>, 0>), r.g, r.b, 0, r.st, *r.p);
+        hipLaunchKernelGGL(k_fixed_dipole<S64A>, r.g, r.b, 0, r.st, *r.p);
         return;
     }
     with_launcher(r, [&](const auto& l) {

@@ -210,35 +210,6 @@ struct Hoisted : Base {
     static constexpr bool kHoist = true;
 };
 
-// a policy whose fields are fixed when the kernel is compiled: B the dipole,
-// E zero (trapped particles in a planetary field).  Its kernel carries no
-// field-kind switch; B is computed by the dipole case of field_f64 /
-// field_f32 itself, so results equal the generic kernel's.
-template <class Base>
-struct DipoleOnly : Base {
-    using R = typename Base::R;
-    __device__ __forceinline__ void eval(const KParams& p, double, R E[3], R B[3]) const
-    {
-        E[0] = E[1] = E[2] = R(0);
-        if constexpr (sizeof(R) == 8) dipole_f64(p.B, this->pos.x, B);
-        else dipole_f32<Base::kFK>(p, p.B, this->pos, B);
-    }
-    template <int ALG>
-    __device__ __forceinline__ void Uf(const KParams& p, const R E[3], const R B[3], const R vin[3], double h,
-                                       R out[3]) const
-    {
-        if constexpr (sizeof(R) == 8 && ALG == 0) boris_f64_sd(vin, E, B, (p.q2m * 0.5) * h, out);
-        else Base::template Uf<ALG>(p, E, B, vin, h, out);
-    }
-    template <int ALG>
-    __device__ __forceinline__ void U(const KParams& p, const R vin[3], double h, double t, R out[3]) const
-    {
-        R E[3], B[3];
-        eval(p, t, E, B);
-        Uf<ALG>(p, E, B, vin, h, out);
-    }
-};
-
 template <class S>
 __device__ __forceinline__ bool outside(const KParams& p, const S& s, const typename S::Pos& xn,
                                         const typename S::R vv[3])

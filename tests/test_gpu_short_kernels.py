@@ -38,3 +38,28 @@ def test_uniform_fields_at_every_remainder(precision, every):
                 kw = dict(dt=dt, savestepinterval=every, save_start=nt % 2 == 0, save_end=nt % 3 == 0)
                 assert_same_bits(prob, precision, **kw)
                 assert_same_bits(prob, precision, **dict(kw, save_everystep=False))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32c"])
+@pytest.mark.parametrize("every", [1, 2, 3, 7])
+def test_dipole_at_every_remainder(precision, every):
+    rng = np.random.default_rng(10 + every)
+    n = 67
+    r = rng.uniform(2.0, 7.0, n) * TP.Re
+    ph = rng.uniform(0.0, 2 * np.pi, n)
+    xv = np.stack([r * np.cos(ph), r * np.sin(ph), rng.uniform(-1.0, 1.0, n) * TP.Re, *rng.normal(0.0, 2e7, (3, n))], 1)
+    xv[::5, 2] = 0.0                  # the equator: two components of B are zero
+    xv[1::5, 5] = -0.0
+    xv[2::7, 3:] = 0.0                # at rest
+    dts = 2 * np.pi * TP.mi / (TP.qi * 3.12e-5 * (TP.Re / r) ** 3) / 32
+    dip = TP.DipoleField(3.12e-5, TP.Re)
+    left = 0
+    for q in (1.0, -1.0):
+        for nt in (1, 2, 3, 4, 9, 60):
+            prob = TP.TraceProblem(xv, (0.0, 0.0), (q * TP.qi / TP.mi, TP.mi, TP.ZeroField(), dip, TP.ZeroField()))
+            for out in (None, TP.InsideSphere(2.5 * TP.Re) | TP.OutsideSphere(6.5 * TP.Re),
+                        TP.InsideSphere(2.5 * TP.Re) | TP.OutsideBox([-6 * TP.Re] * 3, [6 * TP.Re] * 3)):
+                for kw in (dict(savestepinterval=every), dict(save_everystep=False), dict(save_start=False)):
+                    a = assert_same_bits(prob, precision, dts=dts, nsteps=nt, isoutside=out, **kw)
+                    left += int((a.retcodes == 1).sum())
+    assert left > 100
