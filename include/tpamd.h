@@ -147,6 +147,8 @@ typedef struct tpamd_solve_desc {
 
 /* descriptor flags */
 #define TPAMD_FLAG_GENERIC_KERNELS 1  /* skip the specialised kernels (gridded B, uniform fields, the dipole): for cross-checks */
+#define TPAMD_FLAG_GRADIENT_BY_COMPONENT 2  /* tpamd_adjoint: dL_dB as [3][nx][ny][nz] instead of the node layout */
+#define TPAMD_FLAG_CHECKPOINTS 4            /* tpamd_adjoint: checkpoints whatever memory is free */
 
 typedef struct tpamd_stats {
     double kernel_ms;         /* device time of the push kernel, HIP events on the solve stream */
@@ -276,9 +278,12 @@ int32_t tpamd_solve_device(tpamd_ctx* ctx, const tpamd_solve_desc* desc,
  * differentiates with ForwardDiff through the CPU solve (src/utility/utility.jl,
  * test/test_derivatives.jl); there is no reverse-mode counterpart.
  *   desc: alg = BORIS, adaptive = 0, precision FP64 or FP32C, no boundary.
- *   ckpt_interval K: FP64 state checkpoints every K steps; the reverse sweep
- *     recomputes each K-step segment.
- *   targets[N][3]; dL_dB in B's node layout [nz][ny][nx][3] (summed in double);
+ *   ckpt_interval K: where the trajectory takes more than half of the free
+ *     device memory (or with TPAMD_FLAG_CHECKPOINTS), FP64 state checkpoints every
+ *     K steps stand in for it and
+ *     the reverse sweep recomputes each K-step segment.
+ *   targets[N][3]; dL_dB in B's node layout [nz][ny][nx][3] (with
+ *     TPAMD_FLAG_GRADIENT_BY_COMPONENT as [3][nx][ny][nz]), summed in double;
  *   dL_dxv0[N][6].  stats->kernel_ms = forward pass, aux_ms = reverse.
  *   FP32C: forward, recompute and reverse steps in float; the adjoint state
  *   carries a per-particle power-of-two exponent, so gradients far beyond the

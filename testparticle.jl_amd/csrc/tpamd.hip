@@ -92,6 +92,31 @@ int tpamd::fail(tpamd_ctx* ctx, int code, const char* fmt, ...)
     return code;
 }
 
+hipError_t tpamd::ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out)
+{
+    if (bytes > ctx->d_buf_bytes) {
+        if (ctx->d_buf) {
+            const hipError_t e = hipFree(ctx->d_buf);
+            if (e != hipSuccess) return e;
+        }
+        ctx->d_buf = nullptr;
+        ctx->d_buf_bytes = 0;
+        const hipError_t e = hipMalloc(&ctx->d_buf, bytes);
+        if (e != hipSuccess) return e;
+        ctx->d_buf_bytes = bytes;
+    }
+    *out = ctx->d_buf;
+    return hipSuccess;
+}
+
+void tpamd::ctx_trim(tpamd_ctx* ctx)
+{
+    if (ctx->d_buf_bytes <= kKeepBytes) return;
+    (void)hipFree(ctx->d_buf);
+    ctx->d_buf = nullptr;
+    ctx->d_buf_bytes = 0;
+}
+
 namespace {
 
 
@@ -646,6 +671,7 @@ int32_t tpamd_init(int32_t device, tpamd_ctx** out)
     c->scratch = nullptr;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
+        hipEventCreate(&c->ev2) != hipSuccess ||
         hipMalloc((void**)&c->d_steps, sizeof(unsigned long long)) != hipSuccess) {
         delete c;
         return fail(nullptr, TPAMD_ERR_DEVICE, "HIP context set-up failed on device %d", device);
@@ -669,6 +695,7 @@ int32_t tpamd_finalize(tpamd_ctx* ctx)
     (void)hipFree(ctx->d_steps);
     (void)hipEventDestroy(ctx->ev0);
     (void)hipEventDestroy(ctx->ev1);
+    (void)hipEventDestroy(ctx->ev2);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return TPAMD_OK;
@@ -1188,14 +1215,8 @@ int32_t tpamd_solve(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fi
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t need = al(b_xv) + al(b_u) + al(b_t) + 2 * al(b_i) + al(b_dt);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    if (need > ctx->d_buf_bytes) {
-        if (ctx->d_buf) HIP_TRY(ctx, hipFree(ctx->d_buf));
-        ctx->d_buf = nullptr;
-        ctx->d_buf_bytes = 0;
-        HIP_TRY(ctx, hipMalloc(&ctx->d_buf, need));
-        ctx->d_buf_bytes = need;
-    }
-    char* b = (char*)ctx->d_buf;
+    char* b = nullptr;
+    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&b));
     double* d_xv = (double*)b; b += al(b_xv);
     double* d_u = (double*)b; b += al(b_u);
     double* d_t = (double*)b; b += al(b_t);
@@ -1267,7 +1288,8 @@ int32_t tpamd_adjoint(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_
     const bool per = B->d.extrap == kExtrapPeriodic;
     const bool cells = B->d.cells != nullptr;      // gathers from the cell-replicated copy
     return adjoint_launch(ctx, p, B, xv0, N, targets, ckpt_interval, nt, loss, dL_dB, dL_dxv0, stats,
-                          f32, bf32, per, cells);
+                          f32, bf32, per, cells, (desc->flags & TPAMD_FLAG_GRADIENT_BY_COMPONENT) != 0,
+                          (desc->flags & TPAMD_FLAG_CHECKPOINTS) != 0);
 }
 
 int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* E,
@@ -1316,14 +1338,8 @@ int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpa
                  b_u = sizeof(double) * 6 * (size_t)cap * (size_t)N, b_t = sizeof(double) * (size_t)cap * (size_t)N;
     const size_t need = al(b_st) + al(b_it) + 2 * al(b_i) + al(b_sy) + al(b_u) + al(b_t);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    if (need > ctx->d_buf_bytes) {
-        if (ctx->d_buf) HIP_TRY(ctx, hipFree(ctx->d_buf));
-        ctx->d_buf = nullptr;
-        ctx->d_buf_bytes = 0;
-        HIP_TRY(ctx, hipMalloc(&ctx->d_buf, need));
-        ctx->d_buf_bytes = need;
-    }
-    char* b = (char*)ctx->d_buf;
+    char* b = nullptr;
+    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&b));
     FoArgs a;
     a.state = (double*)b; b += al(b_st);
     a.iters = (long long*)b; b += al(b_it);
@@ -1662,14 +1678,8 @@ int32_t tpamd_solve_batch(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t 
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t need = al(b_xv) + al(b_u) + al(b_t) + 2 * al(b_i);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    if (need > ctx->d_buf_bytes) {
-        if (ctx->d_buf) HIP_TRY(ctx, hipFree(ctx->d_buf));
-        ctx->d_buf = nullptr;
-        ctx->d_buf_bytes = 0;
-        HIP_TRY(ctx, hipMalloc(&ctx->d_buf, need));
-        ctx->d_buf_bytes = need;
-    }
-    char* p = (char*)ctx->d_buf;
+    char* p = nullptr;
+    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&p));
     double* d_xv = (double*)p; p += al(b_xv);
     double* d_u = (double*)p; p += al(b_u);
     double* d_t = (double*)p; p += al(b_t);

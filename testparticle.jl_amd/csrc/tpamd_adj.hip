@@ -71,20 +71,64 @@ __device__ __forceinline__ void adj_cellcoord(const KParams& p, const AdjState<F
     }
 }
 
-// a record that adds nothing, keyed to a cell that spreads such records over
-// the bins
-template <typename R>
-__device__ __forceinline__ void adj_zero_record(const AdjParams& a, size_t rec)
-{
-    a.rec_key[rec] = (unsigned)(rec % (size_t)a.ncell);
-    AdjRec<R> v;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        v.bb[k] = (R)0;
-        v.w[k] = (R)0;
+// What the reverse step needs of a state, a row of the trajectory: the
+// weights in its cell, its velocity and the cell.  The sign of a weight tells
+// that a clamped grid is clamped along that axis (weights are never negative).
+template <bool F32, bool PER, typename T, bool CELLS>
+struct AdjCell {
+    using S = AdjState<F32, PER, T, CELLS>;
+    using R = typename S::R;
+    R w[3], sc[3];
+    unsigned key;
+    __device__ __forceinline__ void locate(const KParams& p, const AdjParams& a, const S& s)
+    {
+        int i0[3], i1[3];
+        adj_cellcoord<F32, PER, T, CELLS>(p, s, sc);
+        key = kNoCell;
+        w[0] = w[1] = w[2] = (R)0;
+        if (adj_locate<PER, R>(p.B, sc, i0, i1, w))
+            key = (unsigned)i0[0] + (unsigned)a.nc[0] * ((unsigned)i0[1] + (unsigned)a.nc[1] * (unsigned)i0[2]);
     }
-    if constexpr (sizeof(R) == 4) v.e = 0;
-    ((AdjRec<R>*)a.rec_val)[rec] = v;
+    __device__ __forceinline__ void store(const KParams& p, const AdjParams& a, long long row, long long i,
+                                          const S& s) const
+    {
+        const long long N = p.N;
+        const auto b = gbl((R*)a.rows) + row * kAdjRow * N + i;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            R wd = w[d];
+            if constexpr (!PER) {
+                if (p.B.extrap == kExtrapClamp && !(sc[d] >= (R)0 && sc[d] <= (R)(p.B.n[d] - 1))) wd = -wd;
+            }
+            b[d * N] = wd;
+            b[(3 + d) * N] = s.v[d];
+        }
+        gbl(a.row_key)[row * N + i] = key;
+    }
+};
+
+// One forward step's velocity update U(v, x, h) with its row written on the
+// way.  The cell is loaded first and the row stored behind it: the memory
+// counter completes in order, so a wait for loads issued after the stores
+// would be a wait for the stores too.
+template <bool F32, bool PER, typename T, bool CELLS>
+__device__ __forceinline__ void adj_step_row(const KParams& p, const AdjParams& a, long long row, long long i,
+                                             const AdjState<F32, PER, T, CELLS>& s, double h,
+                                             typename AdjState<F32, PER, T, CELLS>::R out[3])
+{
+    using R = typename AdjState<F32, PER, T, CELLS>::R;
+    AdjCell<F32, PER, T, CELLS> q;
+    q.locate(p, a, s);
+    T raw[24];
+    R c[8][3], B[3];
+    const R E[3] = {(R)0, (R)0, (R)0};
+    if (q.key != kNoCell) adj_corners<T, PER, CELLS>(p.B, a.nc, q.key, raw);
+    q.store(p, a, row, i, s);
+#pragma unroll
+    for (int k = 0; k < 24; ++k) c[k / 3][k % 3] = (R)raw[k];
+    if (q.key != kNoCell) adj_value<R>(c, q.w, B);
+    else B[0] = B[1] = B[2] = (R)__builtin_nan("");
+    s.template Uf<0>(p, E, B, s.v, h, out);
 }
 
 // Float adjoint state: (xbar, ubar) = (xb, ub) * 2^ex.  Rescales the
@@ -107,27 +151,39 @@ __device__ __forceinline__ void adj_renorm(float xb[3], float ub[3], int& ex)
     }
 }
 
-// one reverse step at the state held in s: (xbar, ubar) <- VJP of the step
-// that started there, with rotation factor h and position step dt.  The
-// step's dL/dB contribution goes to record slot `rec` (cell, Bbar, weights).
+// A row on its way to the reverse step: the state and the corner values of
+// its cell, loaded together (the row's key, known ahead, addresses the cell)
+template <bool F32, typename T>
+struct AdjFetch {
+    using R = typename std::conditional<F32, float, double>::type;
+    R row[kAdjRow];
+    T c[24];
+};
+
+// one reverse step at the state of a fetched row: (xbar, ubar) <- VJP of the
+// step that started there, with rotation factor h and position step dt (0 on
+// the row of the initial half-step, which moves no position).  The step's
+// dL/dB contribution is returned (Bbar, weights, exponent).
 template <bool F32, bool PER, typename T, bool CELLS>
-__device__ __forceinline__ void adj_step_back(const KParams& p, const AdjParams& a,
-                                              const AdjState<F32, PER, T, CELLS>& s, const typename AdjState<F32, PER, T, CELLS>::R u[3],
-                                              double h, double dt, typename AdjState<F32, PER, T, CELLS>::R xb[3],
-                                              typename AdjState<F32, PER, T, CELLS>::R ub[3], int& ex,
-                                              bool with_dt, size_t rec)
+__device__ __forceinline__ AdjRec<typename AdjState<F32, PER, T, CELLS>::R>
+adj_step_back(const KParams& p, const AdjFetch<F32, T>& q, double h, double dt, bool with_dt,
+              typename AdjState<F32, PER, T, CELLS>::R xb[3], typename AdjState<F32, PER, T, CELLS>::R ub[3], int& ex)
 {
     using R = typename AdjState<F32, PER, T, CELLS>::R;
-    R sc[3], w[3], c[8][3], B[3];
-    int i0[3], i1[3];
-    unsigned node[8];
-    adj_cellcoord<F32, PER, T, CELLS>(p, s, sc);
-    if (!adj_locate<PER, R>(p.B, sc, i0, i1, w)) {
-        adj_zero_record<R>(a, rec);
-        return;
+    R w[3], c[8][3], B[3], u[3];
+    bool flat[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        flat[d] = false;
+        w[d] = q.row[d];
+        if constexpr (!PER) {
+            flat[d] = copysign((R)1, w[d]) < (R)0;
+            w[d] = fabs(w[d]);
+        }
+        u[d] = q.row[3 + d];
     }
-    if constexpr (CELLS) adj_corners_cell<T, R>(p.B, i0, c);
-    else adj_corners<T, R>(p.B, i0, i1, c, node);
+#pragma unroll
+    for (int k = 0; k < 24; ++k) c[k / 3][k % 3] = (R)q.c[k];
     adj_value<R>(c, w, B);
     const R hh = (R)h;
     R t[3], g[3], tb[3], un[3], Bb[3], xg[3];
@@ -142,18 +198,15 @@ __device__ __forceinline__ void adj_step_back(const KParams& p, const AdjParams&
     adj_xgrad<R>(p.B, c, w, Bb, xg);
     if constexpr (!PER) {
         // outside the node box a clamped field does not change along that axis
-        if (p.B.extrap == kExtrapClamp) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-                if (!(sc[k] >= (R)0 && sc[k] <= (R)(p.B.n[k] - 1))) xg[k] = (R)0;
-        }
+        for (int k = 0; k < 3; ++k)
+            if (flat[k]) xg[k] = (R)0;
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         xb[k] += xg[k];
         ub[k] = un[k];
     }
-    a.rec_key[rec] = (unsigned)i0[0] + (unsigned)a.nc[0] * ((unsigned)i0[1] + (unsigned)a.nc[1] * (unsigned)i0[2]);
     AdjRec<R> v;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -164,10 +217,12 @@ __device__ __forceinline__ void adj_step_back(const KParams& p, const AdjParams&
         v.e = ex;                  // Bbar carries the state's scale at this step
         adj_renorm(xb, ub, ex);
     }
-    ((AdjRec<R>*)a.rec_val)[rec] = v;
+    return v;
 }
 
-template <bool F32, bool PER, typename T, bool CELLS>
+// The forward pass.  ROWS: the whole trajectory, row 0 the initial state and
+// row n + 1 the state before step n; otherwise a checkpoint every K steps.
+template <bool F32, bool PER, typename T, bool CELLS, bool ROWS>
 __global__ void __launch_bounds__(256) k_adj_forward(const KParams p, const AdjParams a)
 {
     using S = AdjState<F32, PER, T, CELLS>;
@@ -180,14 +235,19 @@ __global__ void __launch_bounds__(256) k_adj_forward(const KParams p, const AdjP
         const double dt = p.dt;
         s.set_dt(dt);
         R vt[3];
-        s.template U<0>(p, s.v, -0.5 * dt, p.t0, vt);            // boris.jl:514
+        if constexpr (ROWS) adj_step_row<F32, PER, T, CELLS>(p, a, 0, i, s, -0.5 * dt, vt);   // boris.jl:514
+        else s.template U<0>(p, s.v, -0.5 * dt, p.t0, vt);
 #pragma unroll
         for (int c = 0; c < 3; ++c) s.v[c] = vt[c];
         double t = fma(-0.5, dt, p.t0);
         for (long long n = 0; n < p.nt; ++n) {
-            if (n % a.K == 0) adj_ckpt_store<F32, PER, T, CELLS>(a, p.N, (int)(n / a.K), i, s);
             t += dt;
-            s.template U<0>(p, s.v, dt, t, vt);
+            if constexpr (ROWS) {
+                adj_step_row<F32, PER, T, CELLS>(p, a, n + 1, i, s, dt, vt);
+            } else {
+                if (n % a.K == 0) adj_ckpt_store<F32, PER, T, CELLS>(a, p.N, (int)(n / a.K), i, s);
+                s.template U<0>(p, s.v, dt, t, vt);
+            }
 #pragma unroll
             for (int c = 0; c < 3; ++c) s.v[c] = vt[c];
             typename S::Pos xn;
@@ -208,25 +268,98 @@ __global__ void __launch_bounds__(256) k_adj_forward(const KParams p, const AdjP
     if ((threadIdx.x & 63) == 0) unsafeAtomicAdd(a.loss, lsum / (double)p.N);
 }
 
-// Reverse sweep over segment `seg` (launched for seg = nseg-1 .. 0): reload
-// the adjoint state, recompute the segment from its checkpoint, walk it
-// backwards writing one record per step into rows 0..K-1 of the record
-// buffer (row K holds the t0 half-step on segment 0; unused rows are marked
-// invalid), and store the adjoint state for the next launch.
+// the rows of segment `seg` from its checkpoint (segment 0: the initial state
+// first), for solves whose trajectory is not kept whole
 template <bool F32, bool PER, typename T, bool CELLS>
-__global__ void __launch_bounds__(256) k_adj_reverse(const KParams p, const AdjParams a, int seg)
+__global__ void __launch_bounds__(256) k_adj_rows(const KParams p, const AdjParams a, int seg)
 {
     using S = AdjState<F32, PER, T, CELLS>;
     using R = typename S::R;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.N) return;
-    const long long N = p.N;
+    const long long n0 = (long long)seg * a.K;
+    const int len = (int)((p.nt - n0) < a.K ? (p.nt - n0) : a.K);
     const double dt = p.dt;
-    const double h = (p.q2m * 0.5) * dt;
+    S s;
+    long long row = 0;
+    if (seg == 0) {
+        AdjCell<F32, PER, T, CELLS> q;
+        s.load(p, i);
+        q.locate(p, a, s);
+        q.store(p, a, row++, i, s);
+    }
+    adj_ckpt_load<F32, PER, T, CELLS>(a, p.N, seg, i, s);
+    s.set_dt(dt);
+    R vt[3];
+    for (int j = 0; j < len; ++j) {
+        adj_step_row<F32, PER, T, CELLS>(p, a, row++, i, s, dt, vt);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) s.v[c] = vt[c];
+        typename S::Pos xn;
+        do_step(p, s, s.v, dt, xn);
+        s.pos = xn;
+    }
+}
+
+// dynamic LDS of k_adj_reverse<..., SORT = true>: the records, their keys,
+// every row's place, the bin counters (one past the last) and the scan's wave sums
+template <typename R>
+constexpr size_t adj_lds_bytes(unsigned nbins)
+{
+    const size_t P = AdjPart::part<R>(), T = AdjPart::kThreads;
+    return P * sizeof(AdjRec<R>) + P * sizeof(unsigned) + P * sizeof(unsigned short) +
+           (((size_t)nbins + T) / T * T + T / 64) * sizeof(unsigned);
+}
+
+// Reverse sweep over rows [row0, row0 + nrow) of the row buffer, last row
+// first, one thread per particle.  `top`: the adjoint state starts from the
+// loss, else from the state the launch above left; `start`: the first row is
+// the initial half-step's, and the sweep ends in the gradient.
+//
+// What bounds it: one thread is a chain of steps, but only the VJP's ~250
+// instructions depend on the step before; rows and cells do not.  So D rows
+// are in flight per thread, each as one group of loads (the row and, by its
+// key, the cell), which hides the gather without occupancy: with SORT the
+// records staged in LDS leave one block of 4 waves a CU.  What is left is
+// memory: a row, a line of cells and a record, 188 B a step in FP32C, run at
+// 5.4 TB/s (131,071 particles x 320 steps, 64^3 float cells: 1.46 ms; with
+// the trajectory recomputed and the records sorted by a kernel of their own
+// it was 2.9 ms).  512 threads a block, or half the records a block and two
+// blocks a CU, measured within 5 %.
+//
+// SORT: per pass of S rows the block ranks the rows' cells by bin (LDS
+// counters and a scan), writes every record to its place in LDS and the pass's
+// records out contiguously: block b of the partition is this block's pass.
+// Otherwise record `row * N + i` goes to its own slot (a zero one where there
+// is none).
+template <bool F32, bool PER, typename T, bool CELLS, bool SORT, int D>
+__global__ void __launch_bounds__(AdjPart::kThreads) k_adj_reverse(const KParams p, const AdjParams a, long long row0,
+                                                                   int nrow, int top, int start)
+{
+    using R = typename AdjState<F32, PER, T, CELLS>::R;
+    constexpr int TH = AdjPart::kThreads, P = AdjPart::part<R>(), S = P / TH, NC = kAdjRow;
+    constexpr unsigned kNone = 0xffffu;
+    static_assert(S % D == 0, "the ring divides a pass");
+    extern __shared__ __align__(16) char lds[];
+    AdjRec<R>* sval = (AdjRec<R>*)lds;
+    unsigned* skey = (unsigned*)(sval + P);
+    unsigned short* slot = (unsigned short*)(skey + P);
+    unsigned* cnt = (unsigned*)(slot + P);
+    const int tid = threadIdx.x;
+    const int nb4 = ((int)a.nbins + TH) / TH * TH;           // counters, padded: a multiple of TH
+    unsigned* wsum = cnt + nb4;
+    const long long N = p.N;
+    const long long i = (long long)blockIdx.x * TH + tid;
+    const bool mine = i < N;
+    const double dt = p.dt;
+    const double h = (p.q2m * 0.5) * dt, h0 = (p.q2m * 0.5) * (-0.5 * dt);
     R* st = (R*)a.state;
     R xb[3], ub[3];
     int ex = 0;                                                // float state: scale 2^ex
-    if (seg == a.nseg - 1) {
+    if (!mine) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) xb[c] = ub[c] = (R)0;
+    } else if (top) {
         double x0[3], m = 0.0;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -249,66 +382,132 @@ __global__ void __launch_bounds__(256) k_adj_reverse(const KParams p, const AdjP
         }
         if constexpr (F32) ex = a.state_exp[i];
     }
-    constexpr int NC = F32 ? 9 : 6;
-    R* buf = (R*)a.seg;
-    const long long n0 = (long long)seg * a.K;
-    const int len = (int)((p.nt - n0) < a.K ? (p.nt - n0) : a.K);
-    S s;
-    adj_ckpt_load<F32, PER, T, CELLS>(a, N, seg, i, s);
-    s.set_dt(dt);
-    R vt[3];
-    for (int j = 0; j < len; ++j) {                           // recompute the segment
-        R* b = buf + (size_t)j * NC * N + i;
+    const int passes = (nrow + S - 1) / S;
+    for (int pass = 0; pass < passes; ++pass) {
+        const int last = nrow - 1 - pass * S;                 // this pass: rows last, last - 1, ...
+        const int m = last + 1 < S ? last + 1 : S;
+        const auto keys = gbl((const unsigned*)a.row_key) + (row0 + last) * N + i;
+        unsigned total = 0;
+        if constexpr (SORT) {
+            for (int k = tid; k < nb4; k += TH) cnt[k] = 0u;
+            __syncthreads();
+            unsigned key[S], rank[S];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            if constexpr (F32) {
-                b[(size_t)d * N] = s.pos.hi[d];
-                b[(size_t)(3 + d) * N] = s.pos.lo[d];
-                b[(size_t)(6 + d) * N] = s.v[d];
+            for (int s = 0; s < S; ++s) key[s] = mine && s < m ? keys[-(long long)s * N] : kNoCell;
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                rank[s] = key[s] != kNoCell ? atomicAdd(&cnt[key[s] >> AdjBin::kShift], 1u) : 0u;
+            __syncthreads();
+            // exclusive scan of the counters, nb4 / TH neighbours a thread
+            const int per = nb4 / TH;
+            unsigned sum = 0;
+            for (int k = 0; k < per; ++k) sum += cnt[tid * per + k];
+            unsigned inc = sum;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned v = __shfl_up(inc, off, 64);
+                if ((tid & 63) >= off) inc += v;
+            }
+            if ((tid & 63) == 63) wsum[tid >> 6] = inc;
+            __syncthreads();
+            unsigned base = inc - sum;
+#pragma unroll
+            for (int w = 0; w < TH / 64; ++w) {
+                if (w < (tid >> 6)) base += wsum[w];
+                total += wsum[w];
+            }
+            for (int k = 0; k < per; ++k) {
+                const unsigned v = cnt[tid * per + k];
+                cnt[tid * per + k] = base;
+                base += v;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                unsigned d = kNone;
+                if (key[s] != kNoCell) {
+                    d = cnt[key[s] >> AdjBin::kShift] + rank[s];
+                    skey[d] = key[s];
+                }
+                slot[s * TH + tid] = (unsigned short)d;
+            }
+            // the table: cnt[nbins] holds the total (the padding's counters are empty)
+            const size_t blk = (size_t)blockIdx.x * passes + pass, nblk = (size_t)gridDim.x * passes;
+            for (unsigned k = tid; k < a.nbins; k += TH)
+                gbl(a.seg)[k * nblk + blk] = AdjPart::seg(cnt[k], cnt[k + 1] - cnt[k]);
+            __syncthreads();
+        }
+        // a row's key again, from its place (SORT) or from the rows
+        auto key_of = [&](int s) -> unsigned {
+            if (!mine || s >= m) return kNoCell;
+            if constexpr (SORT) {
+                const unsigned d = slot[s * TH + tid];
+                return d == kNone ? kNoCell : skey[d];
             } else {
-                b[(size_t)d * N] = s.pos.x[d];
-                b[(size_t)(3 + d) * N] = s.v[d];
+                return keys[-(long long)s * N];
+            }
+        };
+        auto fetch = [&](int s, AdjFetch<F32, T>& q) -> unsigned {
+            const unsigned key = key_of(s);
+            if (key != kNoCell) {
+                const auto b = gbl((const R*)a.rows) + (row0 + last - s) * NC * N + i;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) q.row[c] = b[c * N];
+                adj_corners<T, PER, CELLS>(p.B, a.nc, key, q.c);
+            }
+            return key;
+        };
+        AdjFetch<F32, T> ring[D];
+        unsigned rkey[D];
+#pragma unroll
+        for (int s = 0; s < D; ++s) rkey[s] = fetch(s, ring[s]);
+        for (int s0 = 0; s0 < m; s0 += D) {
+#pragma unroll
+            for (int k = 0; k < D; ++k) {
+                const int s = s0 + k;
+                const unsigned key = rkey[k];
+                const bool half = start && last - s == 0;     // the initial half-step's row
+                if (key != kNoCell) {
+                    const AdjRec<R> v = adj_step_back<F32, PER, T, CELLS>(p, ring[k], half ? h0 : h, half ? 0.0 : dt,
+                                                                          !half, xb, ub, ex);
+                    if constexpr (SORT) {
+                        sval[slot[s * TH + tid]] = v;
+                    } else {
+                        gbl(a.rec_key)[(long long)(last - s) * N + i] = key;
+                        ((AdjRec<R>*)a.rec_val)[(long long)(last - s) * N + i] = v;
+                    }
+                } else if (!SORT && mine && s < m) {
+                    // a record that adds nothing, keyed to a cell that spreads such
+                    // records over the bins
+                    const long long r = (long long)(last - s) * N + i;
+                    AdjRec<R> v{};
+                    gbl(a.rec_key)[r] = (unsigned)(r % (long long)a.ncell);
+                    ((AdjRec<R>*)a.rec_val)[r] = v;
+                }
+                rkey[k] = fetch(s + D, ring[k]);
             }
         }
-        s.template U<0>(p, s.v, dt, 0.0, vt);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) s.v[c] = vt[c];
-        typename S::Pos xn;
-        do_step(p, s, s.v, dt, xn);
-        s.pos = xn;
-    }
-    for (int j = a.K - 1; j >= len; --j) adj_zero_record<R>(a, (size_t)j * N + i);
-    for (int j = len - 1; j >= 0; --j) {                      // and walk it backwards
-        const R* b = buf + (size_t)j * NC * N + i;
-        R u[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            if constexpr (F32) {
-                s.pos.hi[d] = b[(size_t)d * N];
-                s.pos.lo[d] = b[(size_t)(3 + d) * N];
-                u[d] = b[(size_t)(6 + d) * N];
-            } else {
-                s.pos.x[d] = b[(size_t)d * N];
-                u[d] = b[(size_t)(3 + d) * N];
-            }
+        if constexpr (SORT) {
+            __syncthreads();
+            const size_t out = ((size_t)blockIdx.x * passes + pass) * P;
+            typedef unsigned U4 __attribute__((ext_vector_type(4)));
+            // P records are a multiple of 16 B, so a last partial vector stays inside
+            const unsigned nv = (total * (unsigned)sizeof(AdjRec<R>) + 15u) / 16u, nk = (total + 3u) / 4u;
+            const auto ov = gbl((U4*)((AdjRec<R>*)a.rec_val + out));
+            const auto ok = gbl((U4*)(a.rec_key + out));
+            for (unsigned k = tid; k < nv; k += TH) ov[k] = ((const U4*)sval)[k];
+            for (unsigned k = tid; k < nk; k += TH) ok[k] = ((const U4*)skey)[k];
+            __syncthreads();                                  // before the next pass writes LDS
         }
-        adj_step_back<F32, PER, T, CELLS>(p, a, s, u, h, dt, xb, ub, ex, true, (size_t)j * N + i);
     }
-    const size_t last = (size_t)a.K * N + i;
-    if (seg == 0) {
-        // the initial back half-step u(-1/2) = U(v0, x0, -dt/2) (boris.jl:514)
-        S s0;
-        s0.load(p, i);
-        R v0[3] = {s0.v[0], s0.v[1], s0.v[2]};
-        adj_step_back<F32, PER, T, CELLS>(p, a, s0, v0, (p.q2m * 0.5) * (-0.5 * dt), 0.0, xb, ub, ex, false,
-                                          last);
+    if (!mine) return;
+    if (start) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             a.grad_xv0[6 * i + c] = ldexp((double)xb[c], ex);
             a.grad_xv0[6 * i + 3 + c] = ldexp((double)ub[c], ex);
         }
     } else {
-        adj_zero_record<R>(a, last);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             st[(size_t)c * N + i] = xb[c];
@@ -316,12 +515,6 @@ __global__ void __launch_bounds__(256) k_adj_reverse(const KParams p, const AdjP
         }
         if constexpr (F32) a.state_exp[i] = ex;
     }
-}
-
-__global__ void k_zero_f32(float* p, long long n)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
 }
 
 __global__ void k_zero_f64(double* p, long long n)
@@ -346,11 +539,12 @@ __global__ void __launch_bounds__(256) k_count_nonfinite(const double* __restric
 template <bool F32, bool PER, typename T, bool CELLS>
 int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* xv0, int64_t N,
                 const double* targets, int K, int64_t nt, double* loss, double* dL_dB,
-                double* dL_dxv0, tpamd_stats* stats)
+                double* dL_dxv0, tpamd_stats* stats, bool bycomp, bool ckpt)
 {
     using R = typename AdjState<F32, PER, T, CELLS>::R;
+    constexpr int TH = AdjPart::kThreads, P = AdjPart::part<R>(), S = P / TH, NC = kAdjRow;
+    constexpr int D = F32 ? 4 : 2;
     const int nseg = (int)((nt + K - 1) / K);
-    const int ncomp = F32 ? 9 : 6;
     const size_t rs = sizeof(R);
     const int nx = B->d.n[0], ny = B->d.n[1], nz = B->d.n[2];
     const size_t nnodes = (size_t)nx * ny * nz;
@@ -361,74 +555,100 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     const double ncell_d = (double)nc[0] * nc[1] * nc[2];
     if (ncell_d >= 1073741824.0) return fail(ctx, TPAMD_ERR_UNSUPPORTED, "the adjoint supports fewer than 2^30 cells");
     const unsigned ncell = (unsigned)ncell_d;
-    const long long M = (long long)(K + 1) * N;              // record rows 0..K
     if ((double)(K + 1) * (double)N >= 2147483648.0)
         return fail(ctx, TPAMD_ERR_CAPACITY, "too many adjoint records: lower the checkpoint interval or N");
-    // records are partitioned on the bin bits [kShift, cellbits) of the cell
-    // index; a grid of one bin needs no partition
-    constexpr int kShift = AdjBin::kShift;
+    const unsigned nbins = (ncell + AdjBin::kCells - 1) / AdjBin::kCells;
+    // the reverse kernel groups the records while its bin counters fit in LDS
+    const bool sort = nbins <= AdjPart::kMaxBins;
+    const int64_t nrows = nt + 1;
+    const long long nblocks = (N + TH - 1) / TH;
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    // bytes of r rows, and of the records of a launch over r rows
+    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    auto row_bytes = [&](int64_t r) { return al(rs * NC * (size_t)r * N) + al(sizeof(unsigned) * (size_t)r * N); };
+    const size_t b_xv = al(sizeof(double) * 6 * N), b_tg = al(sizeof(double) * 3 * N), b_st = al(rs * 6 * (size_t)N),
+                 b_se = al(sizeof(int) * (size_t)N), b_G = al(sizeof(double) * 24 * (size_t)ncell),
+                 b_out = al(sizeof(double) * 3 * nnodes), b_gx = al(sizeof(double) * 6 * N), b_ls = al(sizeof(double)),
+                 b_xf = al(sizeof(double) * 3 * N), b_nf = al(sizeof(unsigned long long));
+    const size_t fixed = b_xv + b_tg + b_st + b_se + b_G + b_out + b_gx + b_ls + b_xf + b_nf;
+    // The whole trajectory where it takes at most half of the free memory (or
+    // less than checkpoints would); then a launch walks as many rows as make
+    // about 2^24 records (some 0.5 GB in float), a multiple of a pass.
+    // Otherwise segments of K steps.
+    size_t mem_free = 0, mem_total = 0;
+    HIP_TRY(ctx, hipMemGetInfo(&mem_free, &mem_total));
+    mem_free += ctx->d_buf_bytes;                            // ours to use again
+    auto rec_slots = [&](int64_t r) {
+        return sort ? (size_t)nblocks * (size_t)((r + S - 1) / S) * P : (size_t)r * (size_t)N;
+    };
+    auto rec_bytes = [&](int64_t r) {
+        return (sort ? 1 : 2) * (al(sizeof(unsigned) * rec_slots(r)) + al(sizeof(AdjRec<R>) * rec_slots(r))) +
+               al(sort ? sizeof(unsigned) * (size_t)nbins * (size_t)nblocks * (size_t)((r + S - 1) / S) : 1);
+    };
+    const int64_t fit = (1LL << 24) / std::max<long long>(nblocks * TH, 1);
+    int64_t rows_launch = std::min<int64_t>(nrows, std::max<int64_t>(sort ? S : 1, fit / S * S));
+    const int64_t rows_seg = std::min<int64_t>(K + 1, nrows);
+    const size_t need_whole = fixed + row_bytes(nrows) + rec_bytes(rows_launch),
+                 need_ckpt = fixed + al(sizeof(double) * 9 * (size_t)nseg * N) + row_bytes(rows_seg) + rec_bytes(rows_seg);
+    const bool whole = !ckpt && (need_whole <= mem_free / 2 || need_whole <= need_ckpt);
+    if (!whole) rows_launch = rows_seg;
+    const size_t slots = rec_slots(rows_launch);
     int cellbits = 0;
     while ((1u << cellbits) < ncell) ++cellbits;
-    const bool partition = cellbits > kShift;
-    const unsigned nbins = (ncell + AdjBin::kCells - 1) / AdjBin::kCells;
-    // the block-local partition while its bin counters fit in LDS, else a radix sort
-    const bool local = partition && nbins <= AdjPart::kMaxBins;
-    const long long nblk = (M + AdjPart::part<R>() - 1) / AdjPart::part<R>();
-    const long long ncnt = local ? (long long)nbins * nblk : 0;
     size_t temp_bytes = 0;
-    HIP_TRY(ctx, hipSetDevice(ctx->device));
-    if (partition && !local)
-        HIP_TRY(ctx, adj_sort_records<R>(nullptr, temp_bytes, nullptr, nullptr, nullptr, nullptr, M, kShift,
-                                         cellbits, ctx->stream));
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t b_xv = al(sizeof(double) * 6 * N), b_tg = al(sizeof(double) * 3 * N),
-                 b_ck = al(sizeof(double) * 9 * (size_t)nseg * N), b_sg = al(rs * ncomp * (size_t)K * N),
-                 b_st = al(rs * 6 * (size_t)N), b_se = al(sizeof(int) * (size_t)N), b_key = al(sizeof(unsigned) * (size_t)M),
-                 b_val = al(sizeof(AdjRec<R>) * (size_t)M), b_tmp = al(std::max<size_t>(temp_bytes, 1)),
-                 b_G = al(sizeof(double) * 24 * (size_t)ncell), b_out = al(sizeof(double) * 3 * nnodes),
-                 b_gx = al(sizeof(double) * 6 * N), b_ls = al(sizeof(double)), b_xf = al(sizeof(double) * 3 * N),
-                 b_cnt = al(sizeof(unsigned) * (size_t)std::max<long long>(ncnt, 1)),
-                 b_nf = al(sizeof(unsigned long long));
-    const size_t total = b_xv + b_tg + b_ck + b_sg + b_st + b_se + b_nf + 2 * b_key + 2 * b_val + b_tmp + b_G + b_out +
-                         b_gx + b_ls + b_xf + 2 * b_cnt;
+    if (!sort)
+        HIP_TRY(ctx, adj_sort_records<R>(nullptr, temp_bytes, nullptr, nullptr, nullptr, nullptr, (long long)slots,
+                                         AdjBin::kShift, cellbits, ctx->stream));
+    const size_t b_ck = whole ? 0 : al(sizeof(double) * 9 * (size_t)nseg * N),
+                 b_rw = al(rs * NC * (size_t)(whole ? nrows : rows_launch) * N),
+                 b_rk = al(sizeof(unsigned) * (size_t)(whole ? nrows : rows_launch) * N),
+                 b_key = al(sizeof(unsigned) * slots), b_val = al(sizeof(AdjRec<R>) * slots),
+                 b_seg = al(sort ? sizeof(unsigned) * (size_t)nbins * (slots / P) : 1), b_tmp = al(std::max<size_t>(temp_bytes, 1));
+    const size_t total = fixed + b_ck + b_rw + b_rk + (sort ? 1 : 2) * (b_key + b_val) + b_seg + b_tmp;
+    // the context's buffer, kept from call to call up to kKeepBytes: an
+    // allocation of this size is tens of microseconds, its release some
+    // hundreds, and now and then either stalls for tens of milliseconds
     char* buf = nullptr;
-    HIP_TRY(ctx, hipMalloc((void**)&buf, total));
+    HIP_TRY(ctx, ctx_buffer(ctx, total, (void**)&buf));
     char* q = buf;
     auto take = [&](size_t n) { char* r = q; q += n; return (void*)r; };
     double* d_xv = (double*)take(b_xv);
     double* d_tg = (double*)take(b_tg);
     AdjParams a;
-    a.ckpt = (double*)take(b_ck);
-    a.seg = take(b_sg);
     a.state = take(b_st);
     a.state_exp = (int*)take(b_se);
-    unsigned long long* d_nf = (unsigned long long*)take(b_nf);
-    unsigned* keys0 = (unsigned*)take(b_key);
-    unsigned* keys1 = (unsigned*)take(b_key);
-    AdjRec<R>* vals0 = (AdjRec<R>*)take(b_val);
-    AdjRec<R>* vals1 = (AdjRec<R>*)take(b_val);
-    void* d_tmp = take(b_tmp);
     double* G = (double*)take(b_G);
     double* d_out = (double*)take(b_out);
     a.grad_xv0 = (double*)take(b_gx);
     a.loss = (double*)take(b_ls);
     a.xfinal = (double*)take(b_xf);
-    unsigned* d_cnt = (unsigned*)take(b_cnt);      // segment starts [bin][block]
-    unsigned* d_off = (unsigned*)take(b_cnt);      // segment counts [bin][block]
+    unsigned long long* d_nf = (unsigned long long*)take(b_nf);
+    a.ckpt = whole ? nullptr : (double*)take(b_ck);
+    a.rows = take(b_rw);
+    a.row_key = (unsigned*)take(b_rk);
+    a.rec_key = (unsigned*)take(b_key);
+    a.rec_val = take(b_val);
+    unsigned* keys1 = sort ? nullptr : (unsigned*)take(b_key);
+    AdjRec<R>* vals1 = sort ? nullptr : (AdjRec<R>*)take(b_val);
+    a.seg = (unsigned*)take(b_seg);
+    void* d_tmp = take(b_tmp);
     a.targets = d_tg;
-    a.rec_key = keys0;
-    a.rec_val = vals0;
     a.K = K;
     a.nseg = nseg;
     a.ncell = ncell;
+    a.nbins = nbins;
     for (int k = 0; k < 3; ++k) a.nc[k] = nc[k];
     p.xv0 = d_xv;
     hipStream_t st = ctx->stream;
-    const dim3 block(256), grid((unsigned)((N + 255) / 256));
+    const dim3 block(256), grid((unsigned)((N + 255) / 256)), rgrid((unsigned)nblocks);
     const long long ng = 24 * (long long)ncell;
+    const size_t lds = sort ? adj_lds_bytes<R>(nbins) : 0;
     float ms_f = 0.f, ms_r = 0.f;
     hipError_t e = hipMemcpyAsync(d_xv, xv0, sizeof(double) * 6 * N, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipMemcpyAsync(d_tg, targets, sizeof(double) * 3 * N, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess && sort)
+        e = hipFuncSetAttribute((const void*)k_adj_reverse<F32, PER, T, CELLS, true, D>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_zero_f64, dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, st, G, ng);
         hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(64), 0, st, a.loss, 1LL);
@@ -436,35 +656,48 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
         e = hipEventRecord(ctx->ev0, st);
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL((k_adj_forward<F32, PER, T, CELLS>), grid, block, 0, st, p, a);
+        if (whole) hipLaunchKernelGGL((k_adj_forward<F32, PER, T, CELLS, true>), grid, block, 0, st, p, a);
+        else hipLaunchKernelGGL((k_adj_forward<F32, PER, T, CELLS, false>), grid, block, 0, st, p, a);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipEventRecord(ctx->ev1, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms_f, ctx->ev0, ctx->ev1);
-    if (e == hipSuccess) e = hipEventRecord(ctx->ev0, st);
-    for (int seg = nseg - 1; seg >= 0 && e == hipSuccess; --seg) {
-        hipLaunchKernelGGL((k_adj_reverse<F32, PER, T, CELLS>), grid, block, 0, st, p, a, seg);
-        e = hipGetLastError();
-        if (e == hipSuccess && local) {
-            e = adj_localsort_records<R>(keys0, vals0, M, nbins, keys1, vals1, d_cnt, d_off, st);
-            if (e == hipSuccess) e = adj_bins_seg<R>(keys1, vals1, d_cnt, d_off, (int)nblk, nbins, ncell, G, st);
-        } else if (e == hipSuccess) {
-            if (partition)
-                e = adj_sort_records<R>(d_tmp, temp_bytes, keys0, keys1, vals0, vals1, M, kShift, cellbits, st);
-            if (e == hipSuccess) {
-                hipLaunchKernelGGL((k_adj_bins<R>), dim3(nbins), dim3(AdjBin::kThreads), 0, st,
-                                   partition ? keys1 : keys0, partition ? vals1 : vals0, M, ncell, G);
-                e = hipGetLastError();
-            }
+    // one launch over rows [row0, row0 + n): the reverse steps, then the bin sums
+    auto sweep = [&](int64_t row0, int n, int top, int start) {
+        if (sort) hipLaunchKernelGGL((k_adj_reverse<F32, PER, T, CELLS, true, D>), rgrid, dim3(TH), lds, st, p, a, (long long)row0, n, top, start);
+        else hipLaunchKernelGGL((k_adj_reverse<F32, PER, T, CELLS, false, D>), rgrid, dim3(TH), 0, st, p, a, (long long)row0, n, top, start);
+        hipError_t r = hipGetLastError();
+        if (r != hipSuccess) return r;
+        if (sort)
+            return adj_bins_seg<R>(a.rec_key, (const AdjRec<R>*)a.rec_val, a.seg, (int)(nblocks * ((n + S - 1) / S)), nbins, ncell, G, st);
+        const long long M = (long long)n * N;
+        r = adj_sort_records<R>(d_tmp, temp_bytes, a.rec_key, keys1, (const AdjRec<R>*)a.rec_val, vals1, M, AdjBin::kShift, cellbits, st);
+        if (r != hipSuccess) return r;
+        hipLaunchKernelGGL((k_adj_bins<R>), dim3(nbins), dim3(AdjBin::kThreads), 0, st, keys1, vals1, M, ncell, G);
+        return hipGetLastError();
+    };
+    if (whole) {
+        for (int64_t end = nrows; end > 0 && e == hipSuccess;) {
+            const int64_t row0 = std::max<int64_t>(0, end - rows_launch);
+            e = sweep(row0, (int)(end - row0), end == nrows, row0 == 0);
+            end = row0;
+        }
+    } else {
+        for (int seg = nseg - 1; seg >= 0 && e == hipSuccess; --seg) {
+            const int64_t len = std::min<int64_t>(K, nt - (int64_t)seg * K);
+            hipLaunchKernelGGL((k_adj_rows<F32, PER, T, CELLS>), grid, block, 0, st, p, a, seg);
+            e = hipGetLastError();
+            if (e == hipSuccess) e = sweep(0, (int)(len + (seg == 0)), seg == nseg - 1, seg == 0);
         }
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_adj_nodes<double>, dim3((unsigned)((nnodes + 255) / 256)), dim3(256), 0, st, G, nx,
-                           ny, nz, nc[0], nc[1], nc[2], PER ? 1 : 0, d_out);
+        const dim3 ngrid((unsigned)((nx + 7) / 8), (unsigned)((ny + 7) / 8), (unsigned)((nz + 7) / 8));
+        if (bycomp)
+            hipLaunchKernelGGL(k_adj_nodes<true>, ngrid, dim3(512), 0, st, G, nx, ny, nz, nc[0], nc[1], nc[2], PER ? 1 : 0, d_out);
+        else
+            hipLaunchKernelGGL(k_adj_nodes<false>, ngrid, dim3(512), 0, st, G, nx, ny, nz, nc[0], nc[1], nc[2], PER ? 1 : 0, d_out);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipEventRecord(ctx->ev1, st);
+    if (e == hipSuccess) e = hipEventRecord(ctx->ev2, st);
     // the outputs are scanned for entries that are not finite (the loss, the
     // node gradient, the initial-state gradient)
     if (e == hipSuccess) {
@@ -475,14 +708,16 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
                            dim3(256), 0, st, a.grad_xv0, (long long)(6 * N), d_nf);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess) e = hipEventElapsedTime(&ms_r, ctx->ev0, ctx->ev1);
     unsigned long long nonfinite = 0;
-    if (e == hipSuccess) e = hipMemcpy(dL_dB, d_out, sizeof(double) * 3 * nnodes, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(dL_dxv0, a.grad_xv0, sizeof(double) * 6 * N, hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(loss, a.loss, sizeof(double), hipMemcpyDeviceToHost);
-    if (e == hipSuccess) e = hipMemcpy(&nonfinite, d_nf, sizeof nonfinite, hipMemcpyDeviceToHost);
-    (void)hipFree(buf);
+    if (e == hipSuccess) e = hipMemcpyAsync(dL_dB, d_out, sizeof(double) * 3 * nnodes, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(dL_dxv0, a.grad_xv0, sizeof(double) * 6 * N, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(loss, a.loss, sizeof(double), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(&nonfinite, d_nf, sizeof nonfinite, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    else (void)hipStreamSynchronize(st);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms_f, ctx->ev0, ctx->ev1);
+    if (e == hipSuccess) e = hipEventElapsedTime(&ms_r, ctx->ev1, ctx->ev2);
+    ctx_trim(ctx);
     if (e != hipSuccess) return fail(ctx, TPAMD_ERR_DEVICE, "adjoint failed: %s", hipGetErrorString(e));
     if (stats) {
         stats->kernel_ms = ms_f;
@@ -508,10 +743,10 @@ namespace tpamd {
 int adjoint_launch(tpamd_ctx* ctx, const KParams& p, const tpamd_field* B, const double* xv0,
                    int64_t N, const double* targets, int K, int64_t nt, double* loss,
                    double* dL_dB, double* dL_dxv0, tpamd_stats* stats, bool f32, bool bf32,
-                   bool per, bool cells)
+                   bool per, bool cells, bool bycomp, bool ckpt)
 {
 #define TPAMD_ADJ(F32_, PER_, T_, CELLS_) \
-    return adjoint_run<F32_, PER_, T_, CELLS_>(ctx, p, B, xv0, N, targets, K, nt, loss, dL_dB, dL_dxv0, stats)
+    return adjoint_run<F32_, PER_, T_, CELLS_>(ctx, p, B, xv0, N, targets, K, nt, loss, dL_dB, dL_dxv0, stats, bycomp, ckpt)
     if (f32) {
         if (cells) {
             if (per) TPAMD_ADJ(true, true, float, true);

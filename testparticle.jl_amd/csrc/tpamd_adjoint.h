@@ -16,17 +16,23 @@
 // The initial back half-step v(-1/2) = U(v0, x0, -dt/2) (boris.jl:514) is
 // differentiated the same way with h = -q2m dt / 4.
 //
-// Memory: FP64 checkpoints of the state every K steps; the reverse sweep
-// recomputes each K-step segment into a per-particle buffer (structure of
-// arrays, particle index fastest) and walks it backwards.
+// Memory: the forward pass writes the state before every step as a row of
+// the trajectory (structure of arrays, particle index fastest; the cell the
+// state lies in beside it), and the reverse sweep reads the rows backwards:
+// 288 GB hold far more steps than a solve has, and a row read costs less
+// than the gather of a step recomputed.  Where the rows would take more than
+// half of the free memory, the forward pass keeps FP64 checkpoints every K
+// steps instead and each K-step segment's rows are recomputed before they
+// are walked.
 //
-// dL/dB without global atomics: each reverse step writes one record (the
-// cell it sampled, Bbar and the three trilinear weights).  Per segment the
-// records are partitioned by cell bin (a block-local sort in LDS, or a radix
-// sort for grids with more bins than its counters hold), and one workgroup
-// per bin sums its records into per-cell corner moments (8 corners x 3
-// components), which it alone adds into the global per-cell gradient.  A
-// last pass folds the per-cell corner moments into the node gradient.
+// dL/dB without global atomics: each reverse step leaves one record (the
+// cell it sampled, Bbar and the three trilinear weights).  The reverse
+// kernel's blocks group their records by cell bin in LDS and write them out
+// so (for grids with more bins than the counters hold it writes them as they
+// come and a radix sort follows), and one workgroup per bin sums its records
+// into per-cell corner moments (8 corners x 3 components), which it alone
+// adds into the global per-cell gradient.  A last pass folds the per-cell
+// corner moments into the node gradient.
 #pragma once
 
 #include "tpamd_grid.h"
@@ -66,30 +72,40 @@ struct AdjBin {
 };
 
 // Partition of the records by bin (key >> kShift), used while the bin
-// counters fit in LDS: each block of kPart consecutive records is sorted by
-// bin in LDS and written back in place (contiguous, coalesced stores), with
-// the count and block-local start of every (bin, block) segment in [bin][block]
-// tables; the bin kernel then reads its bin's segment from every block.  One
-// read and one write of the records, against two radix passes and a global
-// scatter.  Records keep their bin, not their order within a bin (the bin
-// sums are order-free LDS atomics already).
+// counters fit in LDS: a block of the reverse kernel (kThreads particles)
+// walks part() / kThreads rows, ranks their cells by bin from the rows' keys,
+// forms each record in its bin's place in LDS and writes the block's records
+// out contiguously, with the (start, count) of every (bin, block) segment in
+// a [bin][block] table; the bin kernel then reads its bin's segment from every
+// block.  The records are written once and read once.  Records keep their
+// bin, not their order within a bin (the bin sums are order-free already).
 struct AdjPart {
-    static constexpr int kThreads = 1024;
     static constexpr unsigned kMaxBins = 2048;
-    // records per block: the block's records and keys staged in LDS
+    static constexpr int kThreads = 256;
+    // records per block, staged in LDS (112 KiB, 96 KiB)
     template <typename R>
     static constexpr int part() { return sizeof(R) == 4 ? 4096 : 2048; }
+    // a segment's table entry: block-local start and count
+    static __host__ __device__ unsigned seg(unsigned start, unsigned count) { return start | (count << 16); }
+    static __host__ __device__ unsigned seg_start(unsigned e) { return e & 0xffffu; }
+    static __host__ __device__ unsigned seg_count(unsigned e) { return e >> 16; }
 };
+
+constexpr int kAdjRow = 6;                    // values of a trajectory row: weights, velocity
+constexpr unsigned kNoCell = 0xffffffffu;     // the field is NaN there: the step leaves no record
 
 struct AdjParams {
     const double* targets;    // [N][3]
-    double* ckpt;             // [nseg][9][N]: frame position (3), wrap (3), velocity (3)
-    void* seg;                // [K][9 or 6][N] recompute buffer (float or double)
-    void* state;              // [6][N] adjoint state (xbar, ubar) between segment launches
+    double* ckpt;             // [nseg][9][N]: frame position (3), wrap (3), velocity (3), or null
+    void* rows;               // [rows][kAdjRow][N] (float or double)
+    unsigned* row_key;        // [rows][N] their cells
+    void* state;              // [6][N] adjoint state (xbar, ubar) between launches
     int* state_exp;           // [N] its power-of-two exponent (float adjoint state only)
-    unsigned* rec_key;        // [(K + 1) N] record keys: the cell index
-    void* rec_val;            // [(K + 1) N] AdjRec<R>; rows without a step hold a zero record
+    unsigned* rec_key;        // record keys: the cell index
+    void* rec_val;            // AdjRec<R>
+    unsigned* seg;            // [bin][block] table of the partition
     unsigned ncell;           // cells in the grid
+    unsigned nbins;
     double* grad_xv0;         // [N][6]
     double* loss;             // scalar sum
     double* xfinal;           // [N][3] final positions
@@ -154,33 +170,38 @@ __device__ __forceinline__ bool adj_locate(const DevField& f, const R s[3], int 
     return true;
 }
 
-template <typename T, typename R>
-__device__ __forceinline__ void adj_corners(const DevField& f, const int i0[3], const int i1[3],
-                                            R c[8][3], unsigned node[8])
+// the 24 corner values of cell `key` (corner q = (qx, qy, qz) in bits 0..2, 3
+// components each), from the cell-replicated copy or from the nodes
+template <typename T, bool PER, bool CELLS>
+__device__ __forceinline__ void adj_corners(const DevField& f, const int nc[3], unsigned key, T c[24])
 {
-    const unsigned nx = (unsigned)f.n[0], nxy = (unsigned)f.n[0] * (unsigned)f.n[1];
-    const T* base = (const T*)f.data;
+    if constexpr (CELLS) {
+        constexpr int V = 16 / (int)sizeof(T);
+        typedef T Vec __attribute__((ext_vector_type(V)));
+        const auto q = gbl((const Vec*)((const char*)f.cells + f.cell_stride * key));
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        const unsigned id = (unsigned)((q & 1) ? i1[0] : i0[0]) + nx * (unsigned)(((q >> 1) & 1) ? i1[1] : i0[1]) +
-                            nxy * (unsigned)((q >> 2) ? i1[2] : i0[2]);
-        node[q] = id;
-        const T* p = base + 3u * id;
-        c[q][0] = (R)p[0]; c[q][1] = (R)p[1]; c[q][2] = (R)p[2];
-    }
-}
-
-// the 8 corner vectors from the cell-replicated copy (corner q = (qx, qy, qz)
-// in bits 0..2, 3 components each, as the cell builder stores them)
-template <typename T, typename R>
-__device__ __forceinline__ void adj_corners_cell(const DevField& f, const int i0[3], R c[8][3])
-{
-    const T* rec = (const T*)((const char*)f.cells + cell_offset(f, i0));
+        for (int j = 0; j < 24 / V; ++j) {
+            const Vec a = q[j];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        c[q][0] = (R)rec[3 * q];
-        c[q][1] = (R)rec[3 * q + 1];
-        c[q][2] = (R)rec[3 * q + 2];
+            for (int k = 0; k < V; ++k) c[V * j + k] = a[k];
+        }
+    } else {
+        const unsigned r = key / (unsigned)nc[0];
+        const int i0[3] = {(int)(key - r * (unsigned)nc[0]), (int)(r % (unsigned)nc[1]), (int)(r / (unsigned)nc[1])};
+        int i1[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) i1[d] = PER && i0[d] + 1 == f.n[d] ? 0 : i0[d] + 1;
+        const unsigned nx = (unsigned)f.n[0], nxy = (unsigned)f.n[0] * (unsigned)f.n[1];
+        const auto base = gbl((const T*)f.data);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const unsigned id = (unsigned)((q & 1) ? i1[0] : i0[0]) + nx * (unsigned)(((q >> 1) & 1) ? i1[1] : i0[1]) +
+                                nxy * (unsigned)((q >> 2) ? i1[2] : i0[2]);
+            const auto v = base + (size_t)3 * id;
+            c[3 * q] = v[0];
+            c[3 * q + 1] = v[1];
+            c[3 * q + 2] = v[2];
+        }
     }
 }
 
@@ -281,18 +302,19 @@ __global__ void __launch_bounds__(AdjBin::kThreads) k_adj_bins(const unsigned* _
     }
 }
 
-// node gradient [k][j][i][3] from the per-cell corner moments: node (i, j, k)
-// is corner q of cell (i - qx, j - qy, k - qz), wrapped on periodic grids
-template <typename R>
-__global__ void __launch_bounds__(256) k_adj_nodes(const R* __restrict__ G, int nx, int ny, int nz,
+// node gradient from the per-cell corner moments: node (i, j, k) is corner q
+// of cell (i - qx, j - qy, k - qz), wrapped on periodic grids.  One block per
+// 8^3 nodes, so a block's lines of G serve it whole.  BYCOMP false writes
+// [k][j][i][3], true [3][i][j][k]; the threads run along the fastest axis.
+template <bool BYCOMP>
+__global__ void __launch_bounds__(512) k_adj_nodes(const double* __restrict__ G, int nx, int ny, int nz,
                                                    int cx, int cy, int cz, int periodic,
-                                                   R* __restrict__ out)
+                                                   double* __restrict__ out)
 {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long nn = (long long)nx * ny * nz;
-    if (id >= nn) return;
-    const int i = (int)(id % nx), j = (int)((id / nx) % ny), k = (int)(id / ((long long)nx * ny));
-    R acc[3] = {0, 0, 0};
+    const int f = threadIdx.x & 7, m = (threadIdx.x >> 3) & 7, s = threadIdx.x >> 6;
+    const int i = 8 * blockIdx.x + (BYCOMP ? s : f), j = 8 * blockIdx.y + m, k = 8 * blockIdx.z + (BYCOMP ? f : s);
+    if (i >= nx || j >= ny || k >= nz) return;
+    double acc[3] = {0, 0, 0};
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
         int ci = i - (q & 1), cj = j - ((q >> 1) & 1), ck = k - (q >> 2);
@@ -303,14 +325,20 @@ __global__ void __launch_bounds__(256) k_adj_nodes(const R* __restrict__ G, int 
         } else if (ci < 0 || cj < 0 || ck < 0 || ci >= cx || cj >= cy || ck >= cz) {
             continue;
         }
-        const R* g = G + ((size_t)ci + (size_t)cx * ((size_t)cj + (size_t)cy * (size_t)ck)) * 24 + 3 * q;
+        const double* g = G + ((size_t)ci + (size_t)cx * ((size_t)cj + (size_t)cy * (size_t)ck)) * 24 + 3 * q;
         acc[0] += g[0];
         acc[1] += g[1];
         acc[2] += g[2];
     }
-    out[3 * id] = acc[0];
-    out[3 * id + 1] = acc[1];
-    out[3 * id + 2] = acc[2];
+    if constexpr (BYCOMP) {
+        const size_t nn = (size_t)nx * ny * nz, id = ((size_t)i * ny + j) * nz + k;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) out[c * nn + id] = acc[c];
+    } else {
+        const size_t id = ((size_t)k * ny + j) * nx + i;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) out[3 * id + c] = acc[c];
+    }
 }
 
 }  // namespace tpamd

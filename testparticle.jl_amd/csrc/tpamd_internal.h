@@ -24,9 +24,9 @@ struct tpamd_field {
 struct tpamd_ctx {
     int device;
     hipStream_t stream;
-    hipEvent_t ev0, ev1;
+    hipEvent_t ev0, ev1, ev2;
     std::string err;
-    // staging buffers for tpamd_solve (grown on demand)
+    // device buffer of the calls that stage or need workspace (ctx_buffer)
     void* d_buf;
     size_t d_buf_bytes;
     unsigned long long* d_steps;
@@ -43,16 +43,17 @@ hipError_t adj_sort_records(void* d_temp, size_t& temp_bytes, const unsigned* ke
                             unsigned* keys_out, const AdjRec<R>* vals_in, AdjRec<R>* vals_out,
                             long long n, int begin_bit, int end_bit, hipStream_t stream);
 
-// tpamd_sort.hip: the bin sums over block-sorted records
+// tpamd_sort.hip: the bin sums over the reverse kernel's blocks of records
 template <typename R>
-hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsigned* seg_start,
-                        const unsigned* seg_count, int nblk, unsigned nbins, unsigned ncell,
-                        double* G, hipStream_t stream);
-// tpamd_sort.hip: block-local sort of the records by bin (see AdjPart)
-template <typename R>
-hipError_t adj_localsort_records(const unsigned* keys_in, const AdjRec<R>* vals_in, long long M,
-                                 unsigned nbins, unsigned* keys_out, AdjRec<R>* vals_out,
-                                 unsigned* seg_start, unsigned* seg_count, hipStream_t stream);
+hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsigned* seg, int nblk,
+                        unsigned nbins, unsigned ncell, double* G, hipStream_t stream);
+
+// The context's device buffer, grown to `bytes` (contents are lost): for use
+// within one call, which the caller serialises and which ends synchronised.
+hipError_t ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out);
+// releases it when it has grown past what is kept between calls
+constexpr size_t kKeepBytes = (size_t)4 << 30;
+void ctx_trim(tpamd_ctx* ctx);
 
 // records the message on ctx (or as the last tpamd_init error) and returns code
 int fail(tpamd_ctx* ctx, int code, const char* fmt, ...);
@@ -128,7 +129,7 @@ void launch_fo_segment(const KParams& p, const FoArgs& a, int fk, hipStream_t st
 int adjoint_launch(tpamd_ctx* ctx, const KParams& p, const tpamd_field* B, const double* xv0,
                    int64_t N, const double* targets, int K, int64_t nt, double* loss,
                    double* dL_dB, double* dL_dxv0, tpamd_stats* stats, bool f32, bool bf32,
-                   bool per, bool cells);
+                   bool per, bool cells, bool bycomp, bool ckpt);
 
 }  // namespace tpamd
 

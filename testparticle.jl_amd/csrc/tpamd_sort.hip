@@ -1,8 +1,7 @@
-// tpamd_sort.hip -- partitions of the adjoint's dL/dB records by cell bin:
-// the block-local LDS sort (with hipCUB's block scan) and the radix sort
-// (hipCUB over rocPRIM) for grids with more bins, kept in their own
-// translation unit so that the pusher source does not carry rocPRIM's
-// templates.
+// tpamd_sort.hip -- the bin sums of the adjoint's dL/dB records (with hipCUB's
+// block scan) and the radix sort (hipCUB over rocPRIM) for grids with more
+// bins than the reverse kernel's counters hold, kept in their own translation
+// unit so that the pusher source does not carry rocPRIM's templates.
 #include <hip/hip_runtime.h>
 
 #include <hipcub/hipcub.hpp>
@@ -24,65 +23,6 @@ hipError_t adj_sort_records(void* d_temp, size_t& temp_bytes, const unsigned* ke
 
 namespace {
 
-// Sorts each block of P = AdjPart::part<R>() consecutive records by bin in
-// LDS and writes it back in place; seg_start / seg_count[bin][block] get the
-// block-local start and the count of each bin's segment.
-template <typename R>
-__global__ void __launch_bounds__(AdjPart::kThreads) k_adj_localsort(
-    const unsigned* __restrict__ keys_in, const AdjRec<R>* __restrict__ vals_in, long long M,
-    unsigned nbins, unsigned* __restrict__ keys_out, AdjRec<R>* __restrict__ vals_out,
-    unsigned* __restrict__ seg_start, unsigned* __restrict__ seg_count)
-{
-    constexpr int T = AdjPart::kThreads;
-    constexpr int P = AdjPart::part<R>();
-    constexpr int PER = P / T;                 // records per thread
-    constexpr int BPT = AdjPart::kMaxBins / T; // bin counters per thread in the scan
-    using Scan = hipcub::BlockScan<unsigned, T>;
-    __shared__ typename Scan::TempStorage scan_tmp;
-    __shared__ unsigned cnt[AdjPart::kMaxBins];
-    __shared__ unsigned start[AdjPart::kMaxBins];
-    __shared__ unsigned skey[P];
-    __shared__ AdjRec<R> sval[P];
-    const int tid = threadIdx.x;
-    const long long r0 = (long long)blockIdx.x * P;
-    const int n = (int)(M - r0 < P ? M - r0 : P);
-    for (int i = tid; i < (int)AdjPart::kMaxBins; i += T) cnt[i] = 0u;
-    __syncthreads();
-    unsigned key[PER], rank[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int idx = tid + j * T;
-        key[j] = idx < n ? keys_in[r0 + idx] : 0u;
-        rank[j] = idx < n ? atomicAdd(&cnt[key[j] >> AdjBin::kShift], 1u) : 0u;
-    }
-    __syncthreads();
-    unsigned c[BPT], sc[BPT];
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) c[q] = cnt[tid * BPT + q];
-    Scan(scan_tmp).ExclusiveSum(c, sc);
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) start[tid * BPT + q] = sc[q];
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int idx = tid + j * T;
-        if (idx < n) {
-            const unsigned lp = start[key[j] >> AdjBin::kShift] + rank[j];
-            skey[lp] = key[j];
-            sval[lp] = vals_in[r0 + idx];
-        }
-    }
-    __syncthreads();
-    for (int idx = tid; idx < n; idx += T) {
-        keys_out[r0 + idx] = skey[idx];
-        vals_out[r0 + idx] = sval[idx];
-    }
-    for (unsigned b = tid; b < nbins; b += T) {
-        seg_start[(size_t)b * gridDim.x + blockIdx.x] = start[b];
-        seg_count[(size_t)b * gridDim.x + blockIdx.x] = cnt[b];
-    }
-}
-
 // Index of the f-th record of a bin's concatenated segments within a chunk
 // of blocks starting at block c0: pre[] is the exclusive scan of the
 // segment counts and beg[] the segments' block-local starts (nb entries).
@@ -100,7 +40,7 @@ __device__ __forceinline__ long long seg_record(const unsigned* pre, const unsig
 }
 
 // The sums of k_adj_bins, over block-sorted records: bin b's records are the
-// segments [blk * P + seg_start[b][blk], + seg_count[b][blk]) of every block.
+// segments [blk * P + start, + count) of every block (seg[b][blk]).
 // The bin's row of segment counts is scanned in LDS, kChunk blocks at a time,
 // and thread f takes the f-th record of the concatenated segments, so
 // neighbouring threads read neighbouring records of a segment.
@@ -120,8 +60,7 @@ __device__ __forceinline__ long long seg_record(const unsigned* pre, const unsig
 template <typename R>
 __global__ void __launch_bounds__(AdjBin::kThreads) k_adj_bins_seg(
     const unsigned* __restrict__ keys, const AdjRec<R>* __restrict__ vals,
-    const unsigned* __restrict__ seg_start, const unsigned* __restrict__ seg_count, int nblk,
-    unsigned ncell, double* __restrict__ G)
+    const unsigned* __restrict__ seg, int nblk, unsigned ncell, double* __restrict__ G)
 {
     constexpr int T = AdjBin::kThreads;
     constexpr int kCells = AdjBin::kCells;
@@ -161,11 +100,12 @@ __global__ void __launch_bounds__(AdjBin::kThreads) k_adj_bins_seg(
     const size_t row = (size_t)blockIdx.x * (size_t)nblk;
     for (int c0 = 0; c0 < nblk; c0 += kChunk) {
         const int nb = nblk - c0 < kChunk ? nblk - c0 : kChunk;
-        unsigned v[IPT];
+        unsigned e[IPT], v[IPT];
 #pragma unroll
         for (int q = 0; q < IPT; ++q) {
             const int i = tid * IPT + q;
-            v[q] = i < nb ? seg_count[row + c0 + i] : 0u;
+            e[q] = i < nb ? seg[row + c0 + i] : 0u;
+            v[q] = AdjPart::seg_count(e[q]);
         }
         unsigned total;
         __syncthreads();                      // the previous chunk is done with pre / beg
@@ -174,7 +114,7 @@ __global__ void __launch_bounds__(AdjBin::kThreads) k_adj_bins_seg(
         for (int q = 0; q < IPT; ++q) {
             const int i = tid * IPT + q;
             pre[i] = v[q];
-            beg[i] = i < nb ? seg_start[row + c0 + i] : 0u;
+            beg[i] = AdjPart::seg_start(e[q]);
         }
         __syncthreads();
         if constexpr (!OWN) {
@@ -260,39 +200,18 @@ __global__ void __launch_bounds__(AdjBin::kThreads) k_adj_bins_seg(
 
 // Launches k_adj_bins_seg, one workgroup per bin.
 template <typename R>
-hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsigned* seg_start,
-                        const unsigned* seg_count, int nblk, unsigned nbins, unsigned ncell,
-                        double* G, hipStream_t stream)
+hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsigned* seg, int nblk,
+                        unsigned nbins, unsigned ncell, double* G, hipStream_t stream)
 {
     hipLaunchKernelGGL((k_adj_bins_seg<R>), dim3(nbins), dim3(AdjBin::kThreads), 0, stream, keys, vals,
-                       seg_start, seg_count, nblk, ncell, G);
+                       seg, nblk, ncell, G);
     return hipGetLastError();
 }
 
-template hipError_t adj_bins_seg<float>(const unsigned*, const AdjRec<float>*, const unsigned*,
-                                        const unsigned*, int, unsigned, unsigned, double*, hipStream_t);
-template hipError_t adj_bins_seg<double>(const unsigned*, const AdjRec<double>*, const unsigned*,
-                                         const unsigned*, int, unsigned, unsigned, double*, hipStream_t);
-
-// Launches k_adj_localsort over the M records (nbins <= AdjPart::kMaxBins).
-template <typename R>
-hipError_t adj_localsort_records(const unsigned* keys_in, const AdjRec<R>* vals_in, long long M,
-                                 unsigned nbins, unsigned* keys_out, AdjRec<R>* vals_out,
-                                 unsigned* seg_start, unsigned* seg_count, hipStream_t stream)
-{
-    constexpr int P = AdjPart::part<R>();
-    const long long nblk = (M + P - 1) / P;
-    hipLaunchKernelGGL((k_adj_localsort<R>), dim3((unsigned)nblk), dim3(AdjPart::kThreads), 0, stream,
-                       keys_in, vals_in, M, nbins, keys_out, vals_out, seg_start, seg_count);
-    return hipGetLastError();
-}
-
-template hipError_t adj_localsort_records<float>(const unsigned*, const AdjRec<float>*, long long,
-                                                 unsigned, unsigned*, AdjRec<float>*, unsigned*,
-                                                 unsigned*, hipStream_t);
-template hipError_t adj_localsort_records<double>(const unsigned*, const AdjRec<double>*, long long,
-                                                  unsigned, unsigned*, AdjRec<double>*, unsigned*,
-                                                  unsigned*, hipStream_t);
+template hipError_t adj_bins_seg<float>(const unsigned*, const AdjRec<float>*, const unsigned*, int,
+                                        unsigned, unsigned, double*, hipStream_t);
+template hipError_t adj_bins_seg<double>(const unsigned*, const AdjRec<double>*, const unsigned*, int,
+                                         unsigned, unsigned, double*, hipStream_t);
 
 template hipError_t adj_sort_records<float>(void*, size_t&, const unsigned*, unsigned*,
                                             const AdjRec<float>*, AdjRec<float>*, long long, int,

@@ -30,7 +30,7 @@ BND_NAN, BND_SPHERE_IN, BND_SPHERE_OUT, BND_BOX, BND_GRID = 1, 2, 4, 8, 16
 RET_SUCCESS, RET_TERMINATED, RET_MAXITERS = 0, 1, 2
 FO_ENTER, FO_CHECKED = 1, 2                     # tpamd_fo_segment flags in
 FO_CHECK, FO_END, FO_OUTSIDE = 0, 1, 2          # and status out
-FLAG_GENERIC_KERNELS = 1
+FLAG_GENERIC_KERNELS, FLAG_GRADIENT_BY_COMPONENT, FLAG_CHECKPOINTS = 1, 2, 4
 RETCODE_NAMES = {RET_SUCCESS: "Success", RET_TERMINATED: "Terminated", RET_MAXITERS: "MaxIters"}
 
 

@@ -52,15 +52,16 @@ def loss_gradient(prob, *, dt, targets, precision: str = "fp64", ckpt_interval: 
     ctx = _lib.context(device)
     hB = B.handle(ctx)
     loss = np.zeros(1)
-    gB = np.zeros(B.data.shape)            # device node layout [k][j][i][c]
-    gx = np.zeros((N, 6))
+    desc.flags |= _lib.FLAG_GRADIENT_BY_COMPONENT
+    gB = np.empty((3,) + tuple(B.shape))   # every entry is written, also where one is not finite
+    gx = np.empty((N, 6))
     st = _lib.Stats()
     with ctx.lock:
         rc = ctx.L.tpamd_adjoint(ctx.h, C.byref(desc), hB, _lib.dptr(xv0), N, _lib.dptr(tg),
                                  int(ckpt_interval), _lib.dptr(loss), _lib.dptr(gB),
                                  _lib.dptr(gx), C.byref(st))
     ctx.check(rc, st)
-    return AdjointResult(float(loss[0]), np.ascontiguousarray(gB.transpose(3, 2, 1, 0)), gx,
+    return AdjointResult(float(loss[0]), gB, gx,
                          st.kernel_ms, st.aux_ms, st)
 
 
