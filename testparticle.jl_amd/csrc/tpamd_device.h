@@ -75,6 +75,7 @@ struct DevField {
     const void* cells;
     int nc[3];
     unsigned cell_stride;
+    long long snap_cells;    // time-dependent grids: bytes between the snapshots' cells
     // time-dependent grids (kind TimeGrid): nsnap snapshots of the node
     // array, snap_bytes apart from `data`, at sorted times[nsnap]
     const double* times;
@@ -339,6 +340,85 @@ __device__ __forceinline__ double lerp_f64(double a, double b, double w)
     return fma(w, b, (1.0 - w) * a);
 }
 
+__device__ __forceinline__ float lerp_f32(float a, float b, float w)
+{
+    return fmaf(w, b, (1.0f - w) * a);
+}
+
+template <typename T>
+__device__ __forceinline__ auto at(const void* base, unsigned off)
+{
+    return gbl((const T*)((const char*)base + off));
+}
+
+// The cell-replicated block of a cell: 24 values, corner (dx, dy, dz) at
+// 3 * (dx + 2 dy + 4 dz)
+__device__ __forceinline__ unsigned cell_offset(const DevField& f, const int i0[3])
+{
+    return f.cell_stride *
+           ((unsigned)i0[0] + (unsigned)f.nc[0] * ((unsigned)i0[1] + (unsigned)f.nc[1] * (unsigned)i0[2]));
+}
+
+template <typename T>
+__device__ __forceinline__ void cell_load(const void* base, unsigned off, T v[24])
+{
+    if constexpr (sizeof(T) == 4) {
+        const auto q = gbl((const float4*)((const char*)base + off));
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            const float4 a = q[j];
+            v[4 * j] = a.x; v[4 * j + 1] = a.y; v[4 * j + 2] = a.z; v[4 * j + 3] = a.w;
+        }
+    } else {
+        const auto q = gbl((const double2*)((const char*)base + off));
+#pragma unroll
+        for (int j = 0; j < 12; ++j) {
+            const double2 a = q[j];
+            v[2 * j] = a.x; v[2 * j + 1] = a.y;
+        }
+    }
+}
+
+// trilinear blend of a block: lerp along x, then y, then z
+template <typename T, typename OUT>
+__device__ __forceinline__ void cell_blend(const T v[24], const OUT w[3], OUT out[3])
+{
+    OUT c[4][3];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const OUT a = (OUT)v[6 * q + k], b = (OUT)v[6 * q + 3 + k];
+            if constexpr (sizeof(OUT) == 8) c[q][k] = lerp_f64(a, b, w[0]);
+            else c[q][k] = lerp_f32(a, b, w[0]);
+        }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if constexpr (sizeof(OUT) == 8)
+            out[k] = lerp_f64(lerp_f64(c[0][k], c[1][k], w[1]), lerp_f64(c[2][k], c[3][k], w[1]), w[2]);
+        else
+            out[k] = lerp_f32(lerp_f32(c[0][k], c[1][k], w[1]), lerp_f32(c[2][k], c[3][k], w[1]), w[2]);
+    }
+}
+
+template <typename T, typename OUT>
+__device__ __forceinline__ void trilinear_cell(const void* base, unsigned off, const OUT w[3], OUT out[3])
+{
+    T v[24];
+    cell_load<T>(base, off, v);
+    cell_blend<T, OUT>(v, w, out);
+}
+
+// node array and cells of snapshot k (0 for a static grid)
+__device__ __forceinline__ const void* snapshot(const DevField& f, int k)
+{
+    return (const char*)f.data + (size_t)k * (size_t)f.snap_bytes;
+}
+__device__ __forceinline__ const void* snapshot_cells(const DevField& f, int k)
+{
+    return (const char*)f.cells + (size_t)k * (size_t)f.snap_cells;
+}
+
 __device__ __forceinline__ void node3_f64(const DevField& f, const void* data, long long idx,
                                           double o[3])
 {
@@ -356,11 +436,11 @@ __device__ __forceinline__ void node3_f64(const DevField& f, long long idx, doub
 }
 
 // build_interpolator(CartesianGrid, A::4D, ...) + linear_interp,
-// src/utility/interpolation.jl:119-148, :203-206, :217-235
-__device__ __forceinline__ void grid_f64(const DevField& f, const double x[3], double out[3],
-                                         const void* data = nullptr)
+// src/utility/interpolation.jl:119-148, :203-206, :217-235; from the cells
+// where the field has them (same values, same blend order)
+__device__ __forceinline__ void grid_f64(const DevField& f, const double x[3], double out[3], int snap = 0)
 {
-    const void* base = data ? data : f.data;
+    const void* base = snapshot(f, snap);
     int i0[3], i1[3];
     double w[3];
 #pragma unroll
@@ -395,6 +475,12 @@ __device__ __forceinline__ void grid_f64(const DevField& f, const double x[3], d
             i0[d] = (int)fl;
             i1[d] = i0[d] + 1;
         }
+    }
+    if (f.cells) {
+        const void* cells = snapshot_cells(f, snap);
+        if (f.dtype == 1) trilinear_cell<float, double>(cells, cell_offset(f, i0), w, out);
+        else trilinear_cell<double, double>(cells, cell_offset(f, i0), w, out);
+        return;
     }
     const long long nx = f.n[0], nxy = (long long)f.n[0] * f.n[1];
     double a[3], b[3], c00[3], c10[3], c01[3], c11[3];
@@ -435,11 +521,6 @@ __device__ __forceinline__ int time_bracket(const DevField& f, double t, double&
     if (lo > 0 && lo < f.nsnap) w = (t - f.times[lo - 1]) / (f.times[lo] - f.times[lo - 1]);
     return lo;
 }
-__device__ __forceinline__ const void* snapshot(const DevField& f, int k)
-{
-    return (const char*)f.data + (size_t)k * (size_t)f.snap_bytes;
-}
-
 // Field-kind classes a generic kernel is compiled for: analytic fields only
 // (zero, uniform, affine, dipole), + uniform grids and their time sequences,
 // + meshes (through the out-of-line mesh evaluator).  A solve takes the
@@ -503,12 +584,12 @@ __device__ __forceinline__ void field_f64(const DevField& f, const double x[3], 
             double w;
             const int k = time_bracket(f, t, w);
             if (k == 0 || k >= f.nsnap) {
-                grid_f64(f, x, o, snapshot(f, k == 0 ? 0 : f.nsnap - 1));
+                grid_f64(f, x, o, k == 0 ? 0 : f.nsnap - 1);
                 return;
             }
             double a[3], b[3];
-            grid_f64(f, x, a, snapshot(f, k - 1));
-            grid_f64(f, x, b, snapshot(f, k));
+            grid_f64(f, x, a, k - 1);
+            grid_f64(f, x, b, k);
 #pragma unroll
             for (int c = 0; c < 3; ++c) o[c] = (1.0 - w) * a[c] + w * b[c];   // interpolation.jl:377
             return;
@@ -659,8 +740,8 @@ __device__ __forceinline__ void field_jac_f64(const DevField& f, const double x[
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j) J[i][j] = (1.0 - w) * J1[i][j] + w * J2[i][j];
-        grid_f64(f, x, a, snapshot(f, k - 1));
-        grid_f64(f, x, b, snapshot(f, k));
+        grid_f64(f, x, a, k - 1);
+        grid_f64(f, x, b, k);
         const double dtk = f.times[k] - f.times[k - 1];
 #pragma unroll
         for (int i = 0; i < 3; ++i) dBdt[i] = (b[i] - a[i]) / dtk;
@@ -875,11 +956,6 @@ __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e)
     e = (a - (s - bp)) + (b - bp);
 }
 
-__device__ __forceinline__ float lerp_f32(float a, float b, float w)
-{
-    return fmaf(w, b, (1.0f - w) * a);
-}
-
 template <typename T>
 __device__ __forceinline__ void node3_f32(const T* __restrict__ d, long long idx, float o[3])
 {
@@ -890,8 +966,7 @@ __device__ __forceinline__ void node3_f32(const T* __restrict__ d, long long idx
 // Trilinear gather in float from frame-relative coordinates (frame origin =
 // the grid origin, so s = (hi + lo) / h without cancellation).
 template <typename T>
-__device__ __forceinline__ void grid_f32_t(const DevField& f, const Pos32& x, float out[3],
-                                           const void* data = nullptr)
+__device__ __forceinline__ void grid_f32_t(const DevField& f, const Pos32& x, float out[3], int snap = 0)
 {
     int i0[3], i1[3];
     float w[3];
@@ -927,7 +1002,11 @@ __device__ __forceinline__ void grid_f32_t(const DevField& f, const Pos32& x, fl
             i1[d] = i0[d] + 1;
         }
     }
-    const T* __restrict__ d = (const T*)(data ? data : f.data);
+    if (f.cells) {
+        trilinear_cell<T, float>(snapshot_cells(f, snap), cell_offset(f, i0), w, out);
+        return;
+    }
+    const T* __restrict__ d = (const T*)snapshot(f, snap);
     const long long nx = f.n[0], nxy = (long long)f.n[0] * f.n[1];
     float a[3], b[3], c00[3], c10[3], c01[3], c11[3];
     node3_f32(d, i0[0] + nx * i0[1] + nxy * i0[2], a);
@@ -1046,11 +1125,11 @@ __device__ __forceinline__ void field_f32(const KParams& p, const DevField& f, c
         const int k0 = k == 0 ? 0 : k - 1, k1 = k >= f.nsnap ? f.nsnap - 1 : k;
         float a[3], b[3];
         if (f.dtype == 1) {
-            grid_f32_t<float>(f, x, a, snapshot(f, k0));
-            if (k1 != k0) grid_f32_t<float>(f, x, b, snapshot(f, k1));
+            grid_f32_t<float>(f, x, a, k0);
+            if (k1 != k0) grid_f32_t<float>(f, x, b, k1);
         } else {
-            grid_f32_t<double>(f, x, a, snapshot(f, k0));
-            if (k1 != k0) grid_f32_t<double>(f, x, b, snapshot(f, k1));
+            grid_f32_t<double>(f, x, a, k0);
+            if (k1 != k0) grid_f32_t<double>(f, x, b, k1);
         }
         if (k == 0 || k >= f.nsnap) {
             o[0] = a[0]; o[1] = a[1]; o[2] = a[2];

@@ -16,6 +16,7 @@ struct tpamd_field {
     tpamd::DevField d;
     void* dev_data;          // owned device buffer (grids)
     void* cells_data;        // owned cell-replicated copy (grids, optional)
+    bool cells_off;          // the caller dropped the copy: no solve builds it again
     const tpamd_field* src;  // UxB: the B field it was built from
     size_t bytes;
     tpamd::MeshGrid mesh_host;      // Mesh: host copy of the descriptor (device pointers)
@@ -115,6 +116,10 @@ void launch_spec32(const LaunchReq& r, int emode, int ns, bool per, bool cells);
 // the reference-form multistep classes (ns = kRefBase + n)
 void launch_spec64r(const LaunchReq& r, int emode, int ns, bool per, bool f32, bool cells);
 void launch_spec32r(const LaunchReq& r, int emode, int ns, bool per, bool cells);
+// fixed-step Boris with two gathers a step (tpamd_pair64/32.hip): gridded E
+// and B on one geometry, or (time) B a sequence of snapshots
+void launch_pair64(const LaunchReq& r, bool time, bool uxb, bool per, bool f32, bool cells);
+void launch_pair32(const LaunchReq& r, bool time, bool uxb, bool per, bool cells);
 // full-orbit segments of the hybrid solver (tpamd_hybrid.hip)
 struct FoArgs {
     double* state;       // [N][8] x, v, t, dt

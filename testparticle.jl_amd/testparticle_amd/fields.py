@@ -169,8 +169,10 @@ class GridField(AbstractField):
     (x[i], y[j], z[k]) (Julia's 3 x nx x ny x nz array).  `storage` chooses
     the device storage precision ("f64" or "f32").  `layout="cells"` adds a
     cell-replicated copy on the device (8 corners x 3 components per cell in
-    one block: one cache line per gather for float storage, ~10x the memory);
-    results are identical to `layout="nodes"`."""
+    one block: one cache line per gather for float storage, ~10x the memory)
+    when the field is created; with `layout="nodes"` the first solve with
+    enough gathers to repay it does, if the copy takes less than 1/16 of the
+    free device memory.  Results are identical."""
 
     def __init__(self, A, x, y, z, bc=None, storage=None, layout="nodes"):
         super().__init__()
