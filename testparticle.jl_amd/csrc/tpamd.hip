@@ -117,7 +117,69 @@ void tpamd::ctx_trim(tpamd_ctx* ctx)
     ctx->d_buf_bytes = 0;
 }
 
+hipError_t tpamd::stage_in(tpamd_ctx* ctx, char* dev, size_t span, const HostPart* parts, int n, hipStream_t st)
+{
+    if (span > kStageIn) {
+        for (int k = 0; k < n; ++k) {
+            if (!parts[k].bytes) continue;
+            const hipError_t e =
+                hipMemcpyAsync(dev + parts[k].off, parts[k].host, parts[k].bytes, hipMemcpyHostToDevice, st);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    // an earlier call that failed may have left the piece in flight
+    hipError_t e = hipEventSynchronize(ctx->pin_ev[0]);
+    if (e != hipSuccess) return e;
+    for (int k = 0; k < n; ++k)
+        if (parts[k].bytes) std::memcpy(ctx->h_pin + parts[k].off, parts[k].host, parts[k].bytes);
+    e = hipMemcpyAsync(dev, ctx->h_pin, span, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = hipEventRecord(ctx->pin_ev[0], st);
+    return e;
+}
+
+hipError_t tpamd::stage_out(tpamd_ctx* ctx, const char* dev, size_t span, const HostPart* parts, int n, hipStream_t st)
+{
+    // a quarter of the span, so that a piece is emptied while the next ones
+    // arrive, within limits where a copy's fixed cost does not show
+    const size_t piece =
+        std::min(kPinPiece, std::max((size_t)256 << 10, (span / kPinSlots + 4095) & ~(size_t)4095));
+    const size_t np = (span + piece - 1) / piece;
+    auto issue = [&](size_t k) {
+        const size_t len = std::min(piece, span - k * piece);
+        const int slot = (int)(k % kPinSlots);
+        hipError_t e = hipMemcpyAsync(ctx->h_pin + slot * kPinPiece, dev + k * piece, len, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipEventRecord(ctx->pin_ev[slot], st);
+        return e;
+    };
+    for (size_t k = 0; k < np && k < (size_t)kPinSlots; ++k) {
+        const hipError_t e = issue(k);
+        if (e != hipSuccess) return e;
+    }
+    int first = 0;                                       // first part that ends past the piece's start
+    for (size_t k = 0; k < np; ++k) {
+        const int slot = (int)(k % kPinSlots);
+        hipError_t e = hipEventSynchronize(ctx->pin_ev[slot]);
+        if (e != hipSuccess) return e;
+        const size_t lo = k * piece, hi = std::min(span, lo + piece);
+        while (first < n && parts[first].off + parts[first].bytes <= lo) ++first;
+        for (int m = first; m < n && parts[m].off < hi; ++m) {
+            const size_t a = std::max(lo, parts[m].off), b = std::min(hi, parts[m].off + parts[m].bytes);
+            if (a < b)
+                std::memcpy((char*)parts[m].host + (a - parts[m].off), ctx->h_pin + slot * kPinPiece + (a - lo), b - a);
+        }
+        if (k + kPinSlots < np) {
+            e = issue(k + kPinSlots);
+            if (e != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
+}
+
 namespace {
+
+// the context's pinned word for a step count read back behind a launch
+unsigned long long* pin_word(const tpamd_ctx* ctx) { return (unsigned long long*)(ctx->h_pin + kPinSlots * kPinPiece); }
 
 
 int fill_poly(int n, Poly& P)
@@ -520,13 +582,15 @@ int fill_params(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field*
     return TPAMD_OK;
 }
 
-int solve_impl(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* E,
-               const tpamd_field* B, const double* d_xv0, int64_t N, double* d_out_u,
-               double* d_out_t, int32_t* d_len, int32_t* d_ret, hipStream_t st,
-               tpamd_stats* stats)
+// enqueues the launch between the context's events ev0 and ev1; the kernel
+// adds its steps to *d_steps
+int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* E,
+                  const tpamd_field* B, const double* d_xv0, int64_t N, double* d_out_u,
+                  double* d_out_t, int32_t* d_len, int32_t* d_ret, hipStream_t st,
+                  unsigned long long* d_steps, int64_t& nt, int64_t& nout)
 {
     KParams p;
-    int64_t nt = 0, nout = 0;
+    nt = nout = 0;
     int rc = fill_params(ctx, desc, E, B, d_xv0, N, d_out_u, d_out_t, d_len, d_ret, p, nt, nout);
     if (rc) return rc;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
@@ -538,7 +602,7 @@ int solve_impl(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* 
         p.B = B->d;
         p.E = E->d;
     }
-    HIP_TRY(ctx, hipMemsetAsync(ctx->d_steps, 0, sizeof(unsigned long long), st));
+    p.steps = d_steps;
     const int bs = desc->block_size > 0 ? desc->block_size : 256;
     if (bs % 64 != 0 || bs > 256)
         return fail(ctx, TPAMD_ERR_ARGUMENT, "block_size must be a multiple of 64 up to 256");
@@ -553,7 +617,6 @@ int solve_impl(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* 
         return fail(ctx, TPAMD_ERR_ARGUMENT, "particles_per_lane applies to adaptive solves only");
     const long long ppl = ppl_req > 0 ? ppl_req : std::max(1LL, std::min(8LL, (long long)N / (64LL * 4096)));
     p.span = (int)(64 * ppl);
-    float ms = 0.f;
     if (N > 0) {
         const long long threads = desc->adaptive ? (N + p.span - 1) / p.span * 64 : N;
         const dim3 block(bs), grid((unsigned)((threads + bs - 1) / bs));
@@ -569,9 +632,13 @@ int solve_impl(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* 
         HIP_TRY(ctx, hipGetLastError());
         HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
     }
-    unsigned long long steps = 0;
-    HIP_TRY(ctx, hipMemcpyAsync(&steps, ctx->d_steps, sizeof steps, hipMemcpyDeviceToHost, st));
-    HIP_TRY(ctx, hipStreamSynchronize(st));
+    return TPAMD_OK;
+}
+
+// the figures of an enqueued solve, once the stream has been waited for
+int solve_stats(tpamd_ctx* ctx, int64_t N, unsigned long long steps, int64_t nt, int64_t nout, tpamd_stats* stats)
+{
+    float ms = 0.f;
     if (N > 0) HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     if (stats) {
         stats->kernel_ms = ms;
@@ -770,10 +837,16 @@ int32_t tpamd_init(int32_t device, tpamd_ctx** out)
     c->d_buf = nullptr;
     c->d_buf_bytes = 0;
     c->scratch = nullptr;
+    c->h_pin = nullptr;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&c->stream) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
         hipEventCreate(&c->ev2) != hipSuccess ||
-        hipMalloc((void**)&c->d_steps, sizeof(unsigned long long)) != hipSuccess) {
+        hipMalloc((void**)&c->d_steps, sizeof(unsigned long long)) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_pin, kPinBytes, 0) != hipSuccess ||
+        hipEventCreateWithFlags(&c->pin_ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->pin_ev[1], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->pin_ev[2], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&c->pin_ev[3], hipEventDisableTiming) != hipSuccess) {
         delete c;
         return fail(nullptr, TPAMD_ERR_DEVICE, "HIP context set-up failed on device %d", device);
     }
@@ -794,6 +867,8 @@ int32_t tpamd_finalize(tpamd_ctx* ctx)
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->d_buf) (void)hipFree(ctx->d_buf);
     (void)hipFree(ctx->d_steps);
+    (void)hipHostFree(ctx->h_pin);
+    for (hipEvent_t e : ctx->pin_ev) (void)hipEventDestroy(e);
     (void)hipEventDestroy(ctx->ev0);
     (void)hipEventDestroy(ctx->ev1);
     (void)hipEventDestroy(ctx->ev2);
@@ -1266,7 +1341,15 @@ int32_t tpamd_solve_device(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const t
         return fail(ctx, TPAMD_ERR_ARGUMENT, "null buffer");
     const auto t0 = std::chrono::steady_clock::now();
     hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
-    int rc = solve_impl(ctx, desc, E, B, d_xv0, N, d_out_u, d_out_t, d_out_len, d_retcode, st, stats);
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    int64_t nt = 0, nout = 0;
+    HIP_TRY(ctx, hipMemsetAsync(ctx->d_steps, 0, sizeof(unsigned long long), st));
+    int rc = solve_enqueue(ctx, desc, E, B, d_xv0, N, d_out_u, d_out_t, d_out_len, d_retcode, st, ctx->d_steps, nt, nout);
+    if (rc) return rc;
+    unsigned long long* const steps = pin_word(ctx);
+    HIP_TRY(ctx, hipMemcpyAsync(steps, ctx->d_steps, sizeof *steps, hipMemcpyDeviceToHost, st));
+    HIP_TRY(ctx, hipStreamSynchronize(st));
+    rc = solve_stats(ctx, N, *steps, nt, nout, stats);
     if (rc) return rc;
     if (stats) {
         stats->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1292,32 +1375,33 @@ int32_t tpamd_solve(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fi
     const size_t b_i = sizeof(int32_t) * (size_t)N;
     const size_t b_dt = desc->dt_pp ? sizeof(double) * (size_t)N : 0;
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t need = al(b_xv) + al(b_u) + al(b_t) + 2 * al(b_i) + al(b_dt);
+    // one span: what goes in, the step count, which goes in as zero and comes
+    // back, and what comes out
+    const size_t o_dt = al(b_xv), o_steps = o_dt + al(b_dt), o_u = o_steps + al(sizeof(unsigned long long)),
+                 o_t = o_u + al(b_u), o_len = o_t + al(b_t), o_ret = o_len + al(b_i), need = o_ret + al(b_i);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    char* b = nullptr;
-    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&b));
-    double* d_xv = (double*)b; b += al(b_xv);
-    double* d_u = (double*)b; b += al(b_u);
-    double* d_t = (double*)b; b += al(b_t);
-    int32_t* d_len = (int32_t*)b; b += al(b_i);
-    int32_t* d_ret = (int32_t*)b; b += al(b_i);
-    double* d_dt = (double*)b;
+    char* d = nullptr;
+    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&d));
     hipStream_t st = ctx->stream;
-    if (N > 0) HIP_TRY(ctx, hipMemcpyAsync(d_xv, xv0, b_xv, hipMemcpyHostToDevice, st));
+    unsigned long long steps = 0;
+    const HostPart in[3] = {{const_cast<double*>(xv0), 0, b_xv},
+                            {const_cast<double*>(desc->dt_pp), o_dt, b_dt},
+                            {&steps, o_steps, sizeof steps}};
+    HIP_TRY(ctx, stage_in(ctx, d, o_steps + sizeof steps, in, 3, st));
     tpamd_solve_desc dd = *desc;
-    if (desc->dt_pp && N > 0) {
-        HIP_TRY(ctx, hipMemcpyAsync(d_dt, desc->dt_pp, b_dt, hipMemcpyHostToDevice, st));
-        dd.dt_pp = d_dt;
-    }
-    int rc = solve_impl(ctx, &dd, E, B, d_xv, N, d_u, d_t, d_len, d_ret, st, stats);
+    if (desc->dt_pp && N > 0) dd.dt_pp = (double*)(d + o_dt);
+    int64_t nt = 0, nout = 0;
+    int rc = solve_enqueue(ctx, &dd, E, B, (double*)d, N, (double*)(d + o_u), (double*)(d + o_t), (int32_t*)(d + o_len),
+                           (int32_t*)(d + o_ret), st, (unsigned long long*)(d + o_steps), nt, nout);
     if (rc) return rc;
-    if (N > 0) {
-        if (b_u) HIP_TRY(ctx, hipMemcpyAsync(out_u, d_u, b_u, hipMemcpyDeviceToHost, st));
-        if (b_t) HIP_TRY(ctx, hipMemcpyAsync(out_t, d_t, b_t, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(out_len, d_len, b_i, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(retcode, d_ret, b_i, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipStreamSynchronize(st));
-    }
+    const HostPart out[5] = {{&steps, 0, sizeof steps},
+                             {out_u, o_u - o_steps, b_u},
+                             {out_t, o_t - o_steps, b_t},
+                             {out_len, o_len - o_steps, b_i},
+                             {retcode, o_ret - o_steps, b_i}};
+    if (N > 0) HIP_TRY(ctx, stage_out(ctx, d + o_steps, o_ret + b_i - o_steps, out, 5, st));
+    rc = solve_stats(ctx, N, steps, nt, nout, stats);
+    if (rc) return rc;
     const int64_t ml = N > 0 ? max_len_host(out_len, N) : 0;
     if (stats) {
         stats->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1690,14 +1774,14 @@ int32_t tpamd_batch_run(tpamd_batch* b, void* stream, tpamd_stats* stats)
     HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
     HIP_TRY(ctx, hipGraphLaunch(b->exec, st));
     HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
-    unsigned long long steps = 0;
-    HIP_TRY(ctx, hipMemcpyAsync(&steps, b->d_steps, sizeof steps, hipMemcpyDeviceToHost, st));
+    unsigned long long* const steps = pin_word(ctx);
+    HIP_TRY(ctx, hipMemcpyAsync(steps, b->d_steps, sizeof *steps, hipMemcpyDeviceToHost, st));
     HIP_TRY(ctx, hipStreamSynchronize(st));
     float ms = 0.f;
     HIP_TRY(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
     if (stats) {
         stats->kernel_ms = ms;
-        stats->particle_steps = (int64_t)steps;
+        stats->particle_steps = (int64_t)*steps;
         stats->nt = b->table[0].nt;
         stats->nout = b->table[0].nout;
         stats->max_len = -1;
@@ -1770,7 +1854,8 @@ int32_t tpamd_solve_batch(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t 
     int32_t* d_len = (int32_t*)p; p += al(b_i);
     int32_t* d_ret = (int32_t*)p;
     hipStream_t st = ctx->stream;
-    if (N > 0) HIP_TRY(ctx, hipMemcpyAsync(d_xv, xv0, b_xv, hipMemcpyHostToDevice, st));
+    const HostPart in = {const_cast<double*>(xv0), 0, b_xv};
+    if (N > 0) HIP_TRY(ctx, stage_in(ctx, (char*)d_xv, b_xv, &in, 1, st));
     HIP_TRY(ctx, hipStreamSynchronize(st));
     tpamd_batch* b = nullptr;
     int rc = tpamd_batch_create(ctx, desc, n_inst, E, B, offsets, d_xv, d_u, d_t, d_len, d_ret, &b);
@@ -1778,13 +1863,10 @@ int32_t tpamd_solve_batch(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t 
     rc = tpamd_batch_run(b, st, stats);
     tpamd_batch_free(b);
     if (rc) return rc;
-    if (N > 0) {
-        if (b_u) HIP_TRY(ctx, hipMemcpyAsync(out_u, d_u, b_u, hipMemcpyDeviceToHost, st));
-        if (b_t) HIP_TRY(ctx, hipMemcpyAsync(out_t, d_t, b_t, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(out_len, d_len, b_i, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipMemcpyAsync(retcode, d_ret, b_i, hipMemcpyDeviceToHost, st));
-        HIP_TRY(ctx, hipStreamSynchronize(st));
-    }
+    const size_t o_t = (size_t)((char*)d_t - (char*)d_u), o_len = (size_t)((char*)d_len - (char*)d_u),
+                 o_ret = (size_t)((char*)d_ret - (char*)d_u);
+    const HostPart out[4] = {{out_u, 0, b_u}, {out_t, o_t, b_t}, {out_len, o_len, b_i}, {retcode, o_ret, b_i}};
+    if (N > 0) HIP_TRY(ctx, stage_out(ctx, (char*)d_u, o_ret + b_i, out, 4, st));
     const int64_t ml = N > 0 ? max_len_host(out_len, N) : 0;
     if (stats) {
         stats->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

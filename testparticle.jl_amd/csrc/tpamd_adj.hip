@@ -621,8 +621,8 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     double* d_out = (double*)take(b_out);
     a.grad_xv0 = (double*)take(b_gx);
     a.loss = (double*)take(b_ls);
+    unsigned long long* d_nf = (unsigned long long*)take(b_nf);   // d_out .. d_nf: read back in one span
     a.xfinal = (double*)take(b_xf);
-    unsigned long long* d_nf = (unsigned long long*)take(b_nf);
     a.ckpt = whole ? nullptr : (double*)take(b_ck);
     a.rows = take(b_rw);
     a.row_key = (unsigned*)take(b_rk);
@@ -644,8 +644,9 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     const long long ng = 24 * (long long)ncell;
     const size_t lds = sort ? adj_lds_bytes<R>(nbins) : 0;
     float ms_f = 0.f, ms_r = 0.f;
-    hipError_t e = hipMemcpyAsync(d_xv, xv0, sizeof(double) * 6 * N, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_tg, targets, sizeof(double) * 3 * N, hipMemcpyHostToDevice, st);
+    const HostPart in[2] = {{const_cast<double*>(xv0), 0, sizeof(double) * 6 * N},
+                            {const_cast<double*>(targets), b_xv, sizeof(double) * 3 * N}};
+    hipError_t e = stage_in(ctx, buf, b_xv + sizeof(double) * 3 * N, in, 2, st);
     if (e == hipSuccess && sort)
         e = hipFuncSetAttribute((const void*)k_adj_reverse<F32, PER, T, CELLS, true, D>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -709,10 +710,11 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
         e = hipGetLastError();
     }
     unsigned long long nonfinite = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(dL_dB, d_out, sizeof(double) * 3 * nnodes, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(dL_dxv0, a.grad_xv0, sizeof(double) * 6 * N, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(loss, a.loss, sizeof(double), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(&nonfinite, d_nf, sizeof nonfinite, hipMemcpyDeviceToHost, st);
+    const HostPart out[4] = {{dL_dB, 0, sizeof(double) * 3 * nnodes},
+                             {dL_dxv0, b_out, sizeof(double) * 6 * N},
+                             {loss, b_out + b_gx, sizeof(double)},
+                             {&nonfinite, b_out + b_gx + b_ls, sizeof nonfinite}};
+    if (e == hipSuccess) e = stage_out(ctx, (char*)d_out, b_out + b_gx + b_ls + sizeof nonfinite, out, 4, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     else (void)hipStreamSynchronize(st);
     if (e == hipSuccess) e = hipEventElapsedTime(&ms_f, ctx->ev0, ctx->ev1);
