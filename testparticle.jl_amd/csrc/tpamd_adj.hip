@@ -583,7 +583,7 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     };
     auto rec_bytes = [&](int64_t r) {
         return (sort ? 1 : 2) * (al(sizeof(unsigned) * rec_slots(r)) + al(sizeof(AdjRec<R>) * rec_slots(r))) +
-               al(sort ? sizeof(unsigned) * (size_t)nbins * (size_t)nblocks * (size_t)((r + S - 1) / S) : 1);
+               al(sort ? sizeof(unsigned) * (size_t)nbins * ((size_t)nblocks * (size_t)((r + S - 1) / S) + 1) : 1);
     };
     const int64_t fit = (1LL << 24) / std::max<long long>(nblocks * TH, 1);
     int64_t rows_launch = std::min<int64_t>(nrows, std::max<int64_t>(sort ? S : 1, fit / S * S));
@@ -603,7 +603,8 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
                  b_rw = al(rs * NC * (size_t)(whole ? nrows : rows_launch) * N),
                  b_rk = al(sizeof(unsigned) * (size_t)(whole ? nrows : rows_launch) * N),
                  b_key = al(sizeof(unsigned) * slots), b_val = al(sizeof(AdjRec<R>) * slots),
-                 b_seg = al(sort ? sizeof(unsigned) * (size_t)nbins * (slots / P) : 1), b_tmp = al(std::max<size_t>(temp_bytes, 1));
+                 seg_words = (size_t)nbins * (slots / P),         // and the bins' totals behind them
+                 b_seg = al(sort ? sizeof(unsigned) * (seg_words + nbins) : 1), b_tmp = al(std::max<size_t>(temp_bytes, 1));
     const size_t total = fixed + b_ck + b_rw + b_rk + (sort ? 1 : 2) * (b_key + b_val) + b_seg + b_tmp;
     // the context's buffer, kept from call to call up to kKeepBytes: an
     // allocation of this size is tens of microseconds, its release some
@@ -669,7 +670,7 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
         hipError_t r = hipGetLastError();
         if (r != hipSuccess) return r;
         if (sort)
-            return adj_bins_seg<R>(a.rec_key, (const AdjRec<R>*)a.rec_val, a.seg, (int)(nblocks * ((n + S - 1) / S)), nbins, ncell, G, st);
+            return adj_bins_seg<R>(a.rec_key, (const AdjRec<R>*)a.rec_val, a.seg, a.seg + seg_words, (int)(nblocks * ((n + S - 1) / S)), nbins, ncell, G, st);
         const long long M = (long long)n * N;
         r = adj_sort_records<R>(d_tmp, temp_bytes, a.rec_key, keys1, (const AdjRec<R>*)a.rec_val, vals1, M, AdjBin::kShift, cellbits, st);
         if (r != hipSuccess) return r;

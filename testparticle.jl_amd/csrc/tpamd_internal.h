@@ -49,8 +49,9 @@ hipError_t adj_sort_records(void* d_temp, size_t& temp_bytes, const unsigned* ke
                             long long n, int begin_bit, int end_bit, hipStream_t stream);
 
 // tpamd_sort.hip: the bin sums over the reverse kernel's blocks of records
+// (tot: nbins words of workspace)
 template <typename R>
-hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsigned* seg, int nblk,
+hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsigned* seg, unsigned* tot, int nblk,
                         unsigned nbins, unsigned ncell, double* G, hipStream_t stream);
 
 // The context's device buffer, grown to `bytes` (contents are lost): for use
