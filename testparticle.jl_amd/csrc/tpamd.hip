@@ -1607,7 +1607,15 @@ int32_t tpamd_batch_create(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t
     b->d_counter = nullptr;
     b->d_steps = nullptr;
     b->block_size = desc->block_size > 0 ? desc->block_size : 256;
-    b->ppt = desc->particles_per_lane > 0 ? desc->particles_per_lane : 4;
+    // Adaptive: chunks of 1/2,000 of the particles, within 128 and 2,048: a
+    // wave gets a new parameter block with a chunk of another instance, and
+    // has to wait there for its longest life.  Measured at 2 / 4 / 8 / 16 / 32
+    // a lane, ms: 60,000 particles 0.26 0.28 0.32 0.37 0.49; 1 M (FP64) 0.66
+    // 0.56 0.54 0.61 0.77; 4 M (FP64) 1.41 1.35 1.40 1.28 1.17; 16 M 2.54 2.53
+    // 2.60 2.68 2.49
+    b->ppt = desc->particles_per_lane > 0 ? desc->particles_per_lane
+             : !desc->adaptive            ? 4
+                                          : (int)std::max<int64_t>(2, std::min<int64_t>(32, b->N / 131072));
     b->have_graph = false;
     if (b->block_size % 64 != 0 || b->block_size > 256) {
         tpamd_batch_free(b);

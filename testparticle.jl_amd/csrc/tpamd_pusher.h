@@ -759,63 +759,74 @@ struct S32G : S32C {
 // The batch kernel's work source: the chunks of the kQueues slices, claimed
 // one at a time by a wave.  The chunk index is made wave-uniform
 // (readfirstlane), so the chunk and its instance's parameter block are read
-// with scalar loads.  The index of the chunk after the current one is
-// claimed when the current one is taken (reading the claim later, to overlap
-// the atomic with work, kept a value live through the particle loop and cost
-// 15 VGPRs: 6 waves per SIMD down to 5).  A wave starts on slice
-// blockIdx % kQueues and moves to the next slice once its own is drained.
+// with scalar loads.  A wave claims a chunk when it needs one: one claimed
+// ahead hid the claim, but 4 M particles are 4,000 chunks for 6,000 waves, and
+// half of them found the queue empty (bulk of 4 M particles, one step each:
+// 0.50 ms with, 0.42 ms without at 512 a chunk).  A wave starts on slice
+// blockIdx % kQueues; when that is drained it reads every slice's counter at
+// once, a lane each, and goes to the next open one.
 struct ChunkSource {
     const Chunk* chunks;
     unsigned* counter;
-    int nchunks, lane, j;
-    unsigned q0, q, nq, c, pending;
+    unsigned nchunks, q;
+    int lane;
 
-    __device__ __forceinline__ unsigned claim() const
+    __device__ __forceinline__ unsigned slice_begin(unsigned k) const
     {
-        unsigned v = 0;
-        if (lane == 0) v = atomicAdd(counter + q * kQueueStride, 1u);
-        return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+        return (unsigned)((unsigned long long)nchunks * k / kQueues);
     }
-    __device__ __forceinline__ void open_slice()
-    {
-        q = (q0 + (unsigned)j) % kQueues;
-        nq = (unsigned)nchunks > q ? ((unsigned)nchunks - q + kQueues - 1) / kQueues : 0u;
-        c = claim();
-        pending = c < nq ? claim() : nq;
-    }
+    __device__ __forceinline__ unsigned slice_size(unsigned k) const { return slice_begin(k + 1u) - slice_begin(k); }
     __device__ __forceinline__ void init(const Chunk* ch, unsigned* ctr, int n, int ln)
     {
         chunks = ch;
         counter = ctr;
-        nchunks = n;
+        nchunks = (unsigned)n;
         lane = ln;
-        q0 = blockIdx.x % kQueues;
-        j = 0;
-        open_slice();
+        q = blockIdx.x % kQueues;
     }
     // the next chunk of this wave, false once every slice is drained
     __device__ __forceinline__ bool next(Chunk& out)
     {
-        while (c >= nq) {
-            if (++j >= kQueues) return false;
-            open_slice();
+        while (true) {
+            unsigned c = 0;
+            if (lane == 0) c = atomicAdd(counter + q * kQueueStride, 1u);
+            c = (unsigned)__builtin_amdgcn_readfirstlane((int)c);
+            if (c < slice_size(q)) {
+                out = chunks[slice_begin(q) + c];
+                return true;
+            }
+            const unsigned k = (unsigned)lane % kQueues;
+            const unsigned v = __hip_atomic_load(counter + k * kQueueStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // the open slices, from the next one on (kQueues divides 64)
+            const unsigned long long open = __ballot(v < slice_size(k)) >> ((q + 1u) % kQueues);
+            if (!open) return false;
+            q = (q + 1u + (unsigned)__builtin_ctzll(open)) % kQueues;
         }
-        out = chunks[q + c * kQueues];
-        c = pending;
-        pending = c < nq ? claim() : nq;
-        return true;
     }
 };
 
-// Adaptive particles of every chunk the wave claims: a lane takes the next
-// particle as soon as its own is done (see adaptive_chunk).  Lives are
-// uneven (in a turbulent box most particles leave within a step or two,
-// the longest of a 512-particle chunk lives tens of steps), so when a chunk's
-// last particle has been handed out the wave claims its next chunk at once
-// and keeps feeding idle lanes from it while the old chunk's long-lived
-// particles finish, instead of idling until they do.  That needs the new
-// chunk to be of the same instance (the lanes share one parameter block);
-// a chunk of another instance waits until every lane is done.
+// Adaptive particles of every chunk the wave claims (see adaptive_chunk).
+// Lives are uneven (in a turbulent box most particles leave within a step or
+// two, the longest of 4 M lives 300), so when a chunk's last particle has been
+// handed out the wave claims its next chunk at once and keeps feeding idle
+// lanes from it while the old chunk's long-lived particles finish, instead of
+// idling until they do.  That needs the new chunk to be of the same instance
+// (the lanes share one parameter block); a chunk of another instance waits
+// until every lane is done.
+//
+// What bounds it: 4 M particles are 1.0 GB (0.2 ms), but the longest life is
+// 300 passes of 1.3-1.5 us one after the other, and while a wave finishes and
+// starts particles (records, HBM loads) its pass is far longer.  So lanes that
+// are done wait until kRefill are idle: the records and loads are shared by
+// more particles and the long lives get on in between.  They wait kPatience
+// passes at most, as some lanes may hold particles that never leave.  4 M
+// particles of 24 instances, FP32C, median ms: refilled at once 1.22, at 32
+// idle lanes 1.03, 48 0.99, 56 0.95, 60 0.98; FP64 1.46 -> 1.32; 16 M of 32
+// instances 2.65 -> 2.49; 600,000 with every fifth trapped for 300 steps 1.65,
+// 2.52 without the limit, 1.26 with it.
+constexpr int kRefill = 56;
+constexpr int kPatience = 8;
+
 template <class S, int ALG, bool REC>
 __device__ __forceinline__ long long batch_adaptive(const KParams* __restrict__ table, ChunkSource& src,
                                                     int lane)
@@ -833,13 +844,24 @@ __device__ __forceinline__ long long batch_adaptive(const KParams* __restrict__ 
         long long next = ch.begin, end = ch.end;          // wave-uniform cursor
         bool held = false;                                // nch: claimed, other instance
         bool drained = false;                             // no chunk left to claim
+        bool fin = false;                                 // this lane's particle is to be finished
         bool active = false;
+        int least = kRefill;                              // idle lanes that make a refill worthwhile
+        int patience = kPatience, waited = 0;
         while (true) {
-            if (active && !(r.settle(p) && r.advance(p))) {
-                steps += r.finish(p);
-                active = false;
+            if (active) {
+                if (!(r.settle(p) && r.advance(p))) {
+                    active = false;
+                    fin = true;
+                }
             }
             const unsigned long long idle = __ballot(!active);
+            if (__popcll(idle) < least && ++waited < patience) continue;
+            waited = 0;
+            if (fin) {
+                steps += r.finish(p);
+                fin = false;
+            }
             while (next >= end && !held && !drained) {
                 if (!src.next(nch)) {
                     drained = true;
@@ -851,8 +873,10 @@ __device__ __forceinline__ long long batch_adaptive(const KParams* __restrict__ 
                 }
             }
             if (next >= end) {
-                if (idle != ~0ull) continue;              // running particles still to finish
-                break;
+                if (idle == ~0ull) break;
+                least = 64;                               // running particles still to finish
+                patience = 0x7fffffff;
+                continue;
             }
             if (!active) {
                 const long long idx = next + (long long)__popcll(idle & below);
