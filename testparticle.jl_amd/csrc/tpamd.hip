@@ -472,7 +472,9 @@ void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, hipStrea
         (void)hipGetLastError();
         return;
     }
-    if (build_cells(ctx, f, st) != TPAMD_OK) {                    // solves from the nodes then
+    if (build_cells(ctx, f, st) == TPAMD_OK) {
+        f->cells_auto = true;
+    } else {                                                      // solves from the nodes then
         (void)hipGetLastError();
         ctx->err.clear();
     }
@@ -891,6 +893,7 @@ static int32_t new_field(tpamd_ctx* ctx, tpamd_field** out, int kind)
     f->dev_data = nullptr;
     f->cells_data = nullptr;
     f->cells_off = false;
+    f->cells_auto = false;
     f->src = nullptr;
     f->bytes = 0;
     *out = f;
@@ -1235,13 +1238,18 @@ int32_t tpamd_field_grid_cells(tpamd_ctx* ctx, tpamd_field* f, int32_t enable)
         return fail(ctx, TPAMD_ERR_ARGUMENT, "the cell layout needs a static gridded field");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     if (!enable) {
-        if (f->cells_data) HIP_TRY(ctx, hipFree(f->cells_data));
-        f->cells_data = nullptr;
+        // a batch made since a solve built the copy holds its address, and its
+        // maker asked for no copy: that memory stays with the field
+        if (f->cells_data && !f->cells_auto) {
+            HIP_TRY(ctx, hipFree(f->cells_data));
+            f->cells_data = nullptr;
+        }
         f->d.cells = nullptr;
         f->cells_off = true;
         return TPAMD_OK;
     }
     f->cells_off = false;
+    if (f->cells_data) f->d.cells = f->cells_data;
     if (f->d.cells) return TPAMD_OK;
     if (cells_bytes(f->d) >= 4294967296.0)
         return fail(ctx, TPAMD_ERR_UNSUPPORTED, "cell layout needs fewer than 4 GiB of cells");
