@@ -52,9 +52,11 @@ GATHER_BYTES = {"f32": 8 * 3 * 4, "f64": 8 * 3 * 8}
 # per particle of a solve: its initial state (6 doubles) read, its length and
 # return code (2 x int32) written; per record: x, v (6 doubles) and t
 STATE_BYTES, LEN_BYTES, RECORD_BYTES = 6 * 8, 2 * 4, 7 * 8
-# adjoint reverse sweep per particle-step: 2 gathers + segment state written
-# and read + dL/dB record (key + Bbar + weights) written, read, written, read
-ADJ_REVERSE_BYTES = {"fp32c": 2 * 96 + 2 * 36 + 4 * 32, "fp64": 2 * 192 + 2 * 48 + 4 * 52}
+# adjoint: a trajectory row (cell, weights, velocity), written by the forward
+# pass; the reverse sweep per particle-step reads it, gathers, and has a dL/dB
+# record (key + Bbar + weights) written and read
+ADJ_ROW_BYTES = {"fp32c": 4 + 6 * 4, "fp64": 4 + 6 * 8}
+ADJ_REVERSE_BYTES = {"fp32c": 96 + ADJ_ROW_BYTES["fp32c"] + 2 * 32, "fp64": 192 + ADJ_ROW_BYTES["fp64"] + 2 * 52}
 # algorithmic FLOPs per particle-step (FMA = 2; div, sqrt = 1): standard Boris
 # with E = 0 (37) + position update (6) + dipole evaluation (27)
 DIPOLE_FLOP = 37 + 6 + 27
@@ -253,6 +255,8 @@ def bench_turbulent(args, torch, TP, W, DeviceEnsemble):
             log("[bench] fp64 reference, node layout: uploading and warming up")
             ens = DeviceEnsemble(pn, alg, w.xv0, dt=w.dt, save_everystep=False, precision=prec,
                                  form="reference")
+            # a solve of this length would build the cell copy by itself
+            ens.ctx.check(ens.ctx.L.tpamd_field_grid_cells(ens.ctx.h, ens.hB, 0))
             wall, kms, st = timed_runs(ens.run, torch, 1, 1)
             assert st.particle_steps == N * nsteps, st.particle_steps
             log(f"[bench] fp64 reference, node layout: {wall * 1e3:.1f} ms/solve")
@@ -448,8 +452,7 @@ def bench_dipole(args, torch, TP, W, DeviceEnsemble):
                                          "save_everystep = false, boris.jl:523-551)"},
                      "roofline": {"bound": "valu", "achieved": flops / 1e12, "peak": peak / 1e12,
                                   "unit": "TFLOP/s", "frac": flops / peak,
-                                  "kernel": "k_fixed<DipoleOnly<S64A>, Boris>" if prec == "fp64"
-                                  else "k_fixed<DipoleOnly<S32CA>, Boris>"}}
+                                  "kernel": "k_fixed_dipole<S64A>" if prec == "fp64" else "k_fixed_dipole<S32CA>"}}
         if args.valu:
             # against the FMA rate measured on this GPU (FP32 without packed math)
             meas = args.valu["fp64_fma_flops_per_s" if prec == "fp64" else "fp32_fma_flops_per_s"]
@@ -607,9 +610,9 @@ def bench_adjoint(args, torch, TP, W, DeviceEnsemble):
     out = {"workload": "adjoint_turbulent_64^3", "particles": N, "steps": nsteps,
            "checkpoint_interval": K, "dt": "T_g(B0)/40", "box": "1e7 m periodic",
            "loss": "mean |x(T) - x*|^2",
-           "precisions": {"fp32c": "float storage, forward / recompute / reverse steps in float, FP64 "
-                                   "checkpoints, float adjoint state with a per-particle power-of-two "
-                                   "exponent, dL/dB summed in double",
+           "precisions": {"fp32c": "float storage, forward and reverse steps in float, float "
+                                   "adjoint state with a per-particle power-of-two exponent, "
+                                   "dL/dB summed in double",
                           "fp64": "double storage and arithmetic"}}
     for prec, storage in (("fp32c", "f32"), ("fp64", "f64")):
         # plain forward solve of the same problem, best of both layouts
@@ -636,27 +639,20 @@ def bench_adjoint(args, torch, TP, W, DeviceEnsemble):
         r_ms = float(np.mean([r.reverse_ms for r in rs]))
         best = min(fwd.values())
         g = rs[-1]
-        # the reverse sweep's roofline: per particle-step two gathers
-        # (recompute and reverse), the segment state written and read back,
-        # and the dL/dB record written, sorted (read + write) and summed (read)
+        # the reverse sweep's roofline: per particle-step a row, a gather, and
+        # the dL/dB record written and read
         abytes = ADJ_REVERSE_BYTES[prec]
         psteps = N * nsteps
-        roof = {"bound": "hbm", "kernel": "reverse sweep: k_adj_reverse + k_adj_localsort + k_adj_bins_seg",
+        roof = {"bound": "hbm", "kernel": "reverse sweep: k_adj_reverse + k_adj_bins_seg",
                 "achieved": psteps * abytes / (r_ms * 1e-3) / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                 "frac": psteps * abytes / (r_ms * 1e-3) / HBM_PEAK,
                 "algorithmic_bytes_per_particle_step": abytes, "traffic": None,
                 "forward_frac": psteps * GATHER_BYTES["f32" if prec == "fp32c" else "f64"]
                                 / (best * 1e-3) / HBM_PEAK}
-        prof = os.path.join(ROOT, "profiles", "traffic_adjoint_turbulent_64.json")
-        if os.path.exists(prof):
-            with open(prof) as f:
-                t = json.load(f)
-            roof["traffic"] = psteps * t["kernels"][prec]["total_bytes_per_particle_step"]
-            roof["traffic_source"] = os.path.relpath(prof, ROOT)
         out[prec] = {"forward_solve_ms": fwd, "adjoint_forward_ms": f_ms, "adjoint_reverse_ms": r_ms,
                      "cost_over_forward": (f_ms + r_ms) / best, "roofline": roof,
-                     "cost_floor_by_bytes": (GATHER_BYTES["f32" if prec == "fp32c" else "f64"] + abytes)
-                                            / GATHER_BYTES["f32" if prec == "fp32c" else "f64"],
+                     "cost_floor_by_bytes": (GATHER_BYTES["f32" if prec == "fp32c" else "f64"] + ADJ_ROW_BYTES[prec]
+                                             + abytes) / GATHER_BYTES["f32" if prec == "fp32c" else "f64"],
                      "loss": g.loss,
                      "max_abs_dL_dB": float(np.max(np.abs(g.dL_dB))),
                      "max_abs_dL_dxv0": float(np.max(np.abs(g.dL_dxv0))),
