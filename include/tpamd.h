@@ -229,8 +229,9 @@ int32_t tpamd_field_mesh(tpamd_ctx* ctx, const void* data, int32_t dtype, const 
  * 4 GiB.  Results are unchanged (same values, same blend order).  A solve
  * whose gathers repay it builds the copy by itself where it takes less than
  * 1/16 of the free memory, for this field and for the snapshots of
- * tpamd_field_time_grid, until enable = 0 is asked for once; such a copy's
- * memory is given back with the field. */
+ * tpamd_field_time_grid, until enable = 0 is asked for once.  Batches use
+ * copies that were asked for only.  enable = 0 frees the copy; a batch made
+ * while an asked-for copy was there must not run after that. */
 int32_t tpamd_field_grid_cells(tpamd_ctx* ctx, tpamd_field* f, int32_t enable);
 /* E = -u x B(x) for a uniform drift u; `B` must be the B field of the solve. */
 int32_t tpamd_field_uxb(tpamd_ctx* ctx, const double u[3], const tpamd_field* B,

@@ -685,6 +685,39 @@ struct tpamd_batch {
 
 namespace {
 
+// The parameter blocks of a batch and the kernels it takes: a specialised
+// policy only if every instance maps to the same one.  A cell copy that a
+// solve built by itself is left out: whether the instances' layouts agree
+// decides the policy, and with it the rounding in FP32C, so it may depend on
+// what the caller asked for only, not on which solves ran before.  (So no
+// batch holds the address of such a copy either.)
+int batch_table(tpamd_batch* b, const tpamd_field* const* E, const tpamd_field* const* B, const double* d_xv0,
+                double* d_out_u, double* d_out_t, int32_t* d_len, int32_t* d_ret)
+{
+    const tpamd_solve_desc* desc = &b->desc;
+    int64_t nt, nout;
+    for (int i = 0; i < b->n_inst; ++i) {
+        KParams& p = b->table[i];
+        const int rc = fill_params(b->ctx, desc, E[i], B[i], d_xv0, b->N, d_out_u, d_out_t, d_len, d_ret, p, nt, nout);
+        if (rc) return rc;
+        if (B[i]->cells_auto) p.B.cells = nullptr;
+        if (E[i]->cells_auto) p.E.cells = nullptr;
+    }
+    const KParams& p0 = b->table[0];
+    int em0 = 0;
+    const int ns0 = spec_class(desc, p0, &em0);
+    b->allow_spec = ns0 >= 0;
+    b->fk = kFkAnalytic;
+    for (const KParams& p : b->table) {
+        int em = 0;
+        b->fk = std::max(b->fk, solve_class(p));
+        b->allow_spec = b->allow_spec && spec_class(desc, p, &em) == ns0 && em == em0 && p.B.dtype == p0.B.dtype &&
+                        (p.B.extrap == kExtrapPeriodic) == (p0.B.extrap == kExtrapPeriodic) &&
+                        (p.B.cells != nullptr) == (p0.B.cells != nullptr);
+    }
+    return TPAMD_OK;
+}
+
 // the work chunks of a batch: 64 ppt consecutive particles of one instance,
 // every stride-th of them
 std::vector<Chunk> make_chunks(const std::vector<int64_t>& offsets, int n_inst, int ppt, int stride)
@@ -1238,18 +1271,15 @@ int32_t tpamd_field_grid_cells(tpamd_ctx* ctx, tpamd_field* f, int32_t enable)
         return fail(ctx, TPAMD_ERR_ARGUMENT, "the cell layout needs a static gridded field");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     if (!enable) {
-        // a batch made since a solve built the copy holds its address, and its
-        // maker asked for no copy: that memory stays with the field
-        if (f->cells_data && !f->cells_auto) {
-            HIP_TRY(ctx, hipFree(f->cells_data));
-            f->cells_data = nullptr;
-        }
-        f->d.cells = nullptr;
         f->cells_off = true;
+        f->d.cells = nullptr;
+        f->cells_auto = false;
+        if (f->cells_data) HIP_TRY(ctx, hipFree(f->cells_data));
+        f->cells_data = nullptr;
         return TPAMD_OK;
     }
     f->cells_off = false;
-    if (f->cells_data) f->d.cells = f->cells_data;
+    f->cells_auto = false;               // the caller's from here on
     if (f->d.cells) return TPAMD_OK;
     if (cells_bytes(f->d) >= 4294967296.0)
         return fail(ctx, TPAMD_ERR_UNSUPPORTED, "cell layout needs fewer than 4 GiB of cells");
@@ -1633,27 +1663,10 @@ int32_t tpamd_batch_create(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t
         tpamd_batch_free(b);
         return fail(ctx, TPAMD_ERR_ARGUMENT, "particles_per_lane must be in [0, 1024]");
     }
-    int64_t nt, nout;
-    for (int i = 0; i < n_inst; ++i) {
-        const int rc = fill_params(ctx, desc, E[i], B[i], d_xv0, N, d_out_u, d_out_t, d_out_len,
-                                   d_retcode, b->table[i], nt, nout);
-        if (rc) {
-            tpamd_batch_free(b);
-            return rc;
-        }
-    }
-    // a specialised policy only if every instance maps to the same one
-    int em0 = 0;
-    const int ns0 = spec_class(desc, b->table[0], &em0);
-    b->allow_spec = ns0 >= 0;
-    b->fk = kFkAnalytic;
-    for (int i = 0; i < n_inst; ++i) b->fk = std::max(b->fk, solve_class(b->table[i]));
-    for (int i = 1; i < n_inst && b->allow_spec; ++i) {
-        int em = 0;
-        const int ns = spec_class(desc, b->table[i], &em);
-        b->allow_spec = ns == ns0 && em == em0 && b->table[i].B.dtype == b->table[0].B.dtype &&
-                        (b->table[i].B.extrap == kExtrapPeriodic) == (b->table[0].B.extrap == kExtrapPeriodic) &&
-                        (b->table[i].B.cells != nullptr) == (b->table[0].B.cells != nullptr);
+    int rc = batch_table(b, E, B, d_xv0, d_out_u, d_out_t, d_out_len, d_retcode);
+    if (rc) {
+        tpamd_batch_free(b);
+        return rc;
     }
     hipDeviceProp_t prop;
     hipError_t e = hipSetDevice(ctx->device);
@@ -1670,7 +1683,7 @@ int32_t tpamd_batch_create(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t
     }
     b->d_steps = (unsigned long long*)((char*)b->d_counter + ctr_bytes);
     b->n_cu = prop.multiProcessorCount;
-    int rc = batch_chunks(b, b->ppt, 1);
+    rc = batch_chunks(b, b->ppt, 1);
     if (!rc) rc = batch_capture(b);
     if (rc) {
         tpamd_batch_free(b);
@@ -1717,24 +1730,8 @@ int32_t tpamd_solve_batch_noalloc(tpamd_ctx* ctx, const tpamd_solve_desc* desc, 
     b.block_size = bs;
     b.ppt = ppt;
     b.have_graph = false;
-    int64_t nt, nout;
-    for (int i = 0; i < n_inst; ++i) {
-        const int rc = fill_params(ctx, desc, E[i], B[i], d_xv0, N, d_out_u, d_out_t, d_out_len, d_retcode,
-                                   b.table[i], nt, nout);
-        if (rc) return rc;
-    }
-    int em0 = 0;
-    const int ns0 = spec_class(desc, b.table[0], &em0);
-    b.allow_spec = ns0 >= 0;
-    b.fk = kFkAnalytic;
-    for (int i = 0; i < n_inst; ++i) b.fk = std::max(b.fk, solve_class(b.table[i]));
-    for (int i = 1; i < n_inst && b.allow_spec; ++i) {
-        int em = 0;
-        const int ns = spec_class(desc, b.table[i], &em);
-        b.allow_spec = ns == ns0 && em == em0 && b.table[i].B.dtype == b.table[0].B.dtype &&
-                       (b.table[i].B.extrap == kExtrapPeriodic) == (b.table[0].B.extrap == kExtrapPeriodic) &&
-                       (b.table[i].B.cells != nullptr) == (b.table[0].B.cells != nullptr);
-    }
+    int rc = batch_table(&b, E, B, d_xv0, d_out_u, d_out_t, d_out_len, d_retcode);
+    if (rc) return rc;
     const std::vector<Chunk> ch = make_chunks(b.offsets, n_inst, ppt, 1);
     if ((long long)ch.size() > kNoAllocMaxChunks)
         return fail(ctx, TPAMD_ERR_CAPACITY,
@@ -1760,7 +1757,7 @@ int32_t tpamd_solve_batch_noalloc(tpamd_ctx* ctx, const tpamd_solve_desc* desc, 
     if (!ch.empty())
         HIP_TRY(ctx, hipMemcpyAsync(b.d_chunks, ch.data(), sizeof(Chunk) * ch.size(), hipMemcpyHostToDevice, st));
     HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
-    const int rc = batch_enqueue(&b, st);
+    rc = batch_enqueue(&b, st);
     if (rc) return rc;
     HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
     unsigned long long steps = 0;

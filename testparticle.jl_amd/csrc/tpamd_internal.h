@@ -17,7 +17,7 @@ struct tpamd_field {
     void* dev_data;          // owned device buffer (grids)
     void* cells_data;        // owned cell-replicated copy (grids, optional)
     bool cells_off;          // the caller dropped the copy: no solve builds it again
-    bool cells_auto;         // a solve built it: its memory stays until the field is freed
+    bool cells_auto;         // a solve built it and the caller has not asked for it: no batch uses it
     const tpamd_field* src;  // UxB: the B field it was built from
     size_t bytes;
     tpamd::MeshGrid mesh_host;      // Mesh: host copy of the descriptor (device pointers)
