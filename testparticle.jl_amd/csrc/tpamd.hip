@@ -452,8 +452,10 @@ int build_cells(tpamd_ctx* ctx, tpamd_field* f, hipStream_t st)
 
 // A solve of `gathers` field evaluations from a field's node array builds the
 // cell-replicated copy first, on its stream, where that repays itself within
-// the solve, and the field keeps it (every solve ends synchronised, so later
-// ones find it on any stream).  Measured over grids from 2 MB to 3 GB: a
+// the solve, and the field keeps it.  The copy counts as built at once: the
+// caller has checked its arguments, and leaves, also with an error, only when
+// the stream has been waited for (Drain), so that the next solve finds it on
+// any stream.  Measured over grids from 2 MB to 3 GB: a
 // gather from double nodes reads 4-8 random lines, 1.0-1.6e10 gathers/s, one
 // from cells two, 2.8-6.5e10 (float: 1.2e10 and 5.5-9.9e10); building writes a
 // cell in 0.05 ns, allocating takes some 15 us below 64 MB and 0.05-0.4 ms
@@ -584,8 +586,21 @@ int fill_params(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field*
     return TPAMD_OK;
 }
 
-// enqueues the launch between the context's events ev0 and ev1; the kernel
-// adds its steps to *d_steps
+// Waits for a stream where an entry point is left before it has done so
+// itself: on an error nothing of the call is in flight (a field's copy being
+// built, the caller's host arrays being read).
+struct Drain {
+    hipStream_t st;
+    bool done = false;
+    ~Drain()
+    {
+        if (!done) (void)hipStreamSynchronize(st);
+    }
+};
+
+// Enqueues the launch between the context's events ev0 and ev1; the kernel
+// adds its steps to *d_steps.  Also where it fails it may have enqueued work:
+// the caller drains the stream.
 int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* E,
                   const tpamd_field* B, const double* d_xv0, int64_t N, double* d_out_u,
                   double* d_out_t, int32_t* d_len, int32_t* d_ret, hipStream_t st,
@@ -596,14 +611,6 @@ int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fiel
     int rc = fill_params(ctx, desc, E, B, d_xv0, N, d_out_u, d_out_t, d_len, d_ret, p, nt, nout);
     if (rc) return rc;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    if (!(desc->flags & TPAMD_FLAG_GENERIC_KERNELS)) {
-        // an adaptive particle's steps are not known: two evaluations at least
-        const double gathers = (double)N * (desc->adaptive ? 2.0 : (double)nt + 1.0);
-        offer_cells(ctx, B, gathers, st);
-        if (!p.e_is_uxb) offer_cells(ctx, E, gathers, st);
-        p.B = B->d;
-        p.E = E->d;
-    }
     p.steps = d_steps;
     const int bs = desc->block_size > 0 ? desc->block_size : 256;
     if (bs % 64 != 0 || bs > 256)
@@ -619,6 +626,14 @@ int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fiel
         return fail(ctx, TPAMD_ERR_ARGUMENT, "particles_per_lane applies to adaptive solves only");
     const long long ppl = ppl_req > 0 ? ppl_req : std::max(1LL, std::min(8LL, (long long)N / (64LL * 4096)));
     p.span = (int)(64 * ppl);
+    if (!(desc->flags & TPAMD_FLAG_GENERIC_KERNELS)) {
+        // an adaptive particle's steps are not known: two evaluations at least
+        const double gathers = (double)N * (desc->adaptive ? 2.0 : (double)nt + 1.0);
+        offer_cells(ctx, B, gathers, st);
+        if (!p.e_is_uxb) offer_cells(ctx, E, gathers, st);
+        p.B = B->d;
+        p.E = E->d;
+    }
     if (N > 0) {
         const long long threads = desc->adaptive ? (N + p.span - 1) / p.span * 64 : N;
         const dim3 block(bs), grid((unsigned)((threads + bs - 1) / bs));
@@ -1381,12 +1396,14 @@ int32_t tpamd_solve_device(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const t
     hipStream_t st = stream ? (hipStream_t)stream : ctx->stream;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     int64_t nt = 0, nout = 0;
+    Drain drain{st};
     HIP_TRY(ctx, hipMemsetAsync(ctx->d_steps, 0, sizeof(unsigned long long), st));
     int rc = solve_enqueue(ctx, desc, E, B, d_xv0, N, d_out_u, d_out_t, d_out_len, d_retcode, st, ctx->d_steps, nt, nout);
     if (rc) return rc;
     unsigned long long* const steps = pin_word(ctx);
     HIP_TRY(ctx, hipMemcpyAsync(steps, ctx->d_steps, sizeof *steps, hipMemcpyDeviceToHost, st));
     HIP_TRY(ctx, hipStreamSynchronize(st));
+    drain.done = true;
     rc = solve_stats(ctx, N, *steps, nt, nout, stats);
     if (rc) return rc;
     if (stats) {
@@ -1422,6 +1439,7 @@ int32_t tpamd_solve(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fi
     HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&d));
     hipStream_t st = ctx->stream;
     unsigned long long steps = 0;
+    Drain drain{st};
     const HostPart in[3] = {{const_cast<double*>(xv0), 0, b_xv},
                             {const_cast<double*>(desc->dt_pp), o_dt, b_dt},
                             {&steps, o_steps, sizeof steps}};
@@ -1437,7 +1455,10 @@ int32_t tpamd_solve(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fi
                              {out_t, o_t - o_steps, b_t},
                              {out_len, o_len - o_steps, b_i},
                              {retcode, o_ret - o_steps, b_i}};
-    if (N > 0) HIP_TRY(ctx, stage_out(ctx, d + o_steps, o_ret + b_i - o_steps, out, 5, st));
+    if (N > 0) {
+        HIP_TRY(ctx, stage_out(ctx, d + o_steps, o_ret + b_i - o_steps, out, 5, st));
+        drain.done = true;
+    }
     rc = solve_stats(ctx, N, steps, nt, nout, stats);
     if (rc) return rc;
     const int64_t ml = N > 0 ? max_len_host(out_len, N) : 0;
@@ -1486,16 +1507,24 @@ int32_t tpamd_adjoint(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_
     // with 32-bit byte offsets
     if (3.0 * (bf32 ? 4.0 : 8.0) * (double)B->d.n[0] * (double)B->d.n[1] * (double)B->d.n[2] >= 4294967296.0)
         return fail(ctx, TPAMD_ERR_UNSUPPORTED, "the adjoint needs a node array below 4 GiB");
+    const bool per = B->d.extrap == kExtrapPeriodic;
+    double ncell = 1.0;
+    for (int k = 0; k < 3; ++k) ncell *= (double)(per ? B->d.n[k] : B->d.n[k] - 1);
+    if (ncell >= 1073741824.0) return fail(ctx, TPAMD_ERR_UNSUPPORTED, "the adjoint supports fewer than 2^30 cells");
+    if (((double)ckpt_interval + 1.0) * (double)N >= 2147483648.0)
+        return fail(ctx, TPAMD_ERR_CAPACITY, "too many adjoint records: lower the checkpoint interval or N");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
+    Drain drain{ctx->stream};                       // adjoint_launch leaves early where it fails
     if (bf32 == f32) {                              // the adjoint's kernels on cells
         offer_cells(ctx, B, 2.0 * (double)N * (double)nt, ctx->stream);
         p.B = B->d;
     }
-    const bool per = B->d.extrap == kExtrapPeriodic;
     const bool cells = B->d.cells != nullptr;      // gathers from the cell-replicated copy
-    return adjoint_launch(ctx, p, B, xv0, N, targets, ckpt_interval, nt, loss, dL_dB, dL_dxv0, stats,
-                          f32, bf32, per, cells, (desc->flags & TPAMD_FLAG_GRADIENT_BY_COMPONENT) != 0,
-                          (desc->flags & TPAMD_FLAG_CHECKPOINTS) != 0);
+    rc = adjoint_launch(ctx, p, B, xv0, N, targets, ckpt_interval, nt, loss, dL_dB, dL_dxv0, stats,
+                        f32, bf32, per, cells, (desc->flags & TPAMD_FLAG_GRADIENT_BY_COMPONENT) != 0,
+                        (desc->flags & TPAMD_FLAG_CHECKPOINTS) != 0);
+    drain.done = rc == TPAMD_OK;
+    return rc;
 }
 
 int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_field* E,
@@ -1868,6 +1897,7 @@ int32_t tpamd_solve_batch(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t 
     int32_t* d_ret = (int32_t*)p;
     hipStream_t st = ctx->stream;
     const HostPart in = {const_cast<double*>(xv0), 0, b_xv};
+    Drain drain{st};
     if (N > 0) HIP_TRY(ctx, stage_in(ctx, (char*)d_xv, b_xv, &in, 1, st));
     HIP_TRY(ctx, hipStreamSynchronize(st));
     tpamd_batch* b = nullptr;
@@ -1880,6 +1910,7 @@ int32_t tpamd_solve_batch(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t 
                  o_ret = (size_t)((char*)d_ret - (char*)d_u);
     const HostPart out[4] = {{out_u, 0, b_u}, {out_t, o_t, b_t}, {out_len, o_len, b_i}, {retcode, o_ret, b_i}};
     if (N > 0) HIP_TRY(ctx, stage_out(ctx, (char*)d_u, o_ret + b_i, out, 4, st));
+    drain.done = true;
     const int64_t ml = N > 0 ? max_len_host(out_len, N) : 0;
     if (stats) {
         stats->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -550,13 +550,7 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     const size_t nnodes = (size_t)nx * ny * nz;
     int nc[3];
     for (int k = 0; k < 3; ++k) nc[k] = PER ? B->d.n[k] : B->d.n[k] - 1;
-    if (nc[0] < 1 || nc[1] < 1 || nc[2] < 1)
-        return fail(ctx, TPAMD_ERR_ARGUMENT, "the adjoint's grid needs at least one cell per axis");
-    const double ncell_d = (double)nc[0] * nc[1] * nc[2];
-    if (ncell_d >= 1073741824.0) return fail(ctx, TPAMD_ERR_UNSUPPORTED, "the adjoint supports fewer than 2^30 cells");
-    const unsigned ncell = (unsigned)ncell_d;
-    if ((double)(K + 1) * (double)N >= 2147483648.0)
-        return fail(ctx, TPAMD_ERR_CAPACITY, "too many adjoint records: lower the checkpoint interval or N");
+    const unsigned ncell = (unsigned)nc[0] * (unsigned)nc[1] * (unsigned)nc[2];   // < 2^30
     const unsigned nbins = (ncell + AdjBin::kCells - 1) / AdjBin::kCells;
     // the reverse kernel groups the records while its bin counters fit in LDS
     const bool sort = nbins <= AdjPart::kMaxBins;
@@ -587,7 +581,7 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     };
     const int64_t fit = (1LL << 24) / std::max<long long>(nblocks * TH, 1);
     int64_t rows_launch = std::min<int64_t>(nrows, std::max<int64_t>(sort ? S : 1, fit / S * S));
-    const int64_t rows_seg = std::min<int64_t>(K + 1, nrows);
+    const int64_t rows_seg = std::min<int64_t>((int64_t)K + 1, nrows);
     const size_t need_whole = fixed + row_bytes(nrows) + rec_bytes(rows_launch),
                  need_ckpt = fixed + al(sizeof(double) * 9 * (size_t)nseg * N) + row_bytes(rows_seg) + rec_bytes(rows_seg);
     const bool whole = !ckpt && (need_whole <= mem_free / 2 || need_whole <= need_ckpt);
