@@ -188,15 +188,16 @@ __device__ __forceinline__ void boris_f64(const double v[3], const double E[3], 
     for (int c = 0; c < 3; ++c) out[c] = (vm[c] + vps[c]) + h * E[c];
 }
 
-// x / d for several x over one d, by the instruction sequence of the
+// x / d for several x over one d > 0, by the instruction sequence of the
 // compiler's IEEE double division (reciprocal, two Newton steps on it,
 // quotient, residual, fused correction) with the denominator's half formed
 // once and without its two scaling steps and its fix-up.  Those return
 // their operand unchanged when d and the quotient are normal numbers away
-// from both ends of the exponent range and x is not zero: d in [2^-400,
-// 2^400] and |x| in [2^-512, 2^300] here, so there the quotient is the
-// division's own, bit for bit; callers divide plainly outside (zero x
-// included).
+// from both ends of the exponent range: d in [2^-400, 2^400] and |x| in
+// [2^-512, 2^300] here, so there the quotient is the division's own, bit for
+// bit; callers divide plainly outside.  A zero x keeps its sign, as in the
+// division: the residual is formed with its sign turned, d m - x, and that
+// of a zero x is +0, so the correction subtracts 0.
 struct SharedDiv {
     double d, r;
     __device__ __forceinline__ void init(double den)
@@ -211,7 +212,7 @@ struct SharedDiv {
     __device__ __forceinline__ double div(double x) const
     {
         const double m = x * r;
-        return fma(fma(-d, m, x), r, m);
+        return fma(-fma(d, m, -x), r, m);
     }
 };
 
