@@ -102,7 +102,11 @@ hipError_t tpamd::ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out)
         ctx->d_buf = nullptr;
         ctx->d_buf_bytes = 0;
         const hipError_t e = hipMalloc(&ctx->d_buf, bytes);
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {
+            ctx->d_buf = nullptr;
+            (void)hipGetLastError();                     // or the next launch would report it
+            return e;
+        }
         ctx->d_buf_bytes = bytes;
     }
     *out = ctx->d_buf;
@@ -1519,10 +1523,16 @@ int32_t tpamd_adjoint(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_
         offer_cells(ctx, B, 2.0 * (double)N * (double)nt, ctx->stream);
         p.B = B->d;
     }
-    const bool cells = B->d.cells != nullptr;      // gathers from the cell-replicated copy
-    rc = adjoint_launch(ctx, p, B, xv0, N, targets, ckpt_interval, nt, loss, dL_dB, dL_dxv0, stats,
-                        f32, bf32, per, cells, (desc->flags & TPAMD_FLAG_GRADIENT_BY_COMPONENT) != 0,
-                        (desc->flags & TPAMD_FLAG_CHECKPOINTS) != 0);
+    auto launch = [&](bool ckpt) {
+        const bool cells = p.B.cells != nullptr;    // gathers from the cell-replicated copy
+        return adjoint_launch(ctx, p, B, xv0, N, targets, ckpt_interval, nt, loss, dL_dB, dL_dxv0, stats,
+                              f32, bf32, per, cells, (desc->flags & TPAMD_FLAG_GRADIENT_BY_COMPONENT) != 0, ckpt);
+    };
+    const bool ckpt = (desc->flags & TPAMD_FLAG_CHECKPOINTS) != 0;
+    rc = launch(ckpt);
+    // free memory is a figure of the moment (other processes, and what one
+    // allocation may take at most): the call needs no more than its checkpoints
+    if (rc == TPAMD_ERR_OOM && !ckpt) rc = launch(true);
     drain.done = rc == TPAMD_OK;
     return rc;
 }

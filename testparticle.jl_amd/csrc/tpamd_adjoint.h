@@ -18,12 +18,11 @@
 //
 // Memory: the forward pass writes the state before every step as a row of
 // the trajectory (structure of arrays, particle index fastest; the cell the
-// state lies in beside it), and the reverse sweep reads the rows backwards:
-// 288 GB hold far more steps than a solve has, and a row read costs less
-// than the gather of a step recomputed.  Where the rows would take more than
-// half of the free memory, the forward pass keeps FP64 checkpoints every K
-// steps instead and each K-step segment's rows are recomputed before they
-// are walked.
+// state lies in beside it), and the reverse sweep reads the rows backwards: a
+// row read costs less than the gather of a step recomputed.  Where the rows
+// would take more than the workspace that a context keeps, the forward pass
+// keeps FP64 checkpoints every K steps instead and each K-step segment's rows
+// are recomputed before they are walked.
 //
 // dL/dB without global atomics: each reverse step leaves one record (the
 // cell it sampled, Bbar and the three trilinear weights).  The reverse

@@ -348,15 +348,16 @@ end
 # --- gradients -----------------------------------------------------------------
 """
     loss_gradient(A, xv0; x, y, z, bc = 2, q2m, tspan, dt, targets, precision = :fp64,
-                  ckpt_interval = 64, device = 0) -> (loss, dL_dA, dL_dxv0)
+                  ckpt_interval = 64, checkpoints = false, device = 0) -> (loss, dL_dA, dL_dxv0)
 
 Loss L = mean_i |x_i(T) - x*_i|^2 of the final positions of a fixed-step
 standard Boris solve with E = 0 and B the gridded field A (3 x nx x ny x nz
 on the uniform ranges x, y, z; `bc` 0 fill NaN, 1 clamp, 2 periodic; `cells`
 adds the cell-replicated device copy), and its gradients with respect to every value
 of A and every initial state (xv0 and targets are 6 x N and 3 x N).  One
-forward pass with FP64 checkpoints every `ckpt_interval` steps, then a reverse
-sweep (tpamd_adjoint).  The reference differentiates the same solve with
+forward pass, which keeps the trajectory in device memory where that takes
+less than 4 GiB and otherwise, or with `checkpoints`, a checkpoint every
+`ckpt_interval` steps, then a reverse sweep (tpamd_adjoint).  The reference differentiates the same solve with
 ForwardDiff (test/test_derivatives.jl).  `precision = :fp32c` runs the steps
 in float over float storage.  A loss or gradient that is not finite throws
 a DomainError.
@@ -364,7 +365,7 @@ a DomainError.
 function loss_gradient(A::Array{T, 4}, xv0::AbstractMatrix, targets::AbstractMatrix;
         x::AbstractRange, y::AbstractRange, z::AbstractRange, bc::Integer = 2, q2m::Real,
         tspan, dt::Real, precision::Symbol = :fp64, ckpt_interval::Integer = 64,
-        cells::Bool = true, device::Integer = 0) where {T <: Union{Float32, Float64}}
+        checkpoints::Bool = false, cells::Bool = true, device::Integer = 0) where {T <: Union{Float32, Float64}}
     size(A, 1) == 3 || throw(ArgumentError("A must be 3 x nx x ny x nz"))
     size(xv0, 1) == 6 && size(targets) == (3, size(xv0, 2)) ||
         throw(ArgumentError("xv0 must be 6 x N and targets 3 x N"))
@@ -376,7 +377,8 @@ function loss_gradient(A::Array{T, 4}, xv0::AbstractMatrix, targets::AbstractMat
                               (Ptr{Cvoid}, Ptr{Cvoid}, Int32), ctx, hB, Int32(1)))
     N = size(xv0, 2)
     d = SolveDesc(q2m = q2m, t0 = tspan[1], t1 = tspan[2], dt = dt, save_start = 0,
-                  save_everystep = 0, precision = precision === :fp32c ? 1 : 0, nout_cap = 1)
+                  save_everystep = 0, precision = precision === :fp32c ? 1 : 0, nout_cap = 1,
+                  flags = checkpoints ? 4 : 0)          # TPAMD_FLAG_CHECKPOINTS
     x0 = Matrix{Float64}(xv0)
     tg = Matrix{Float64}(targets)
     loss = Ref(0.0)
