@@ -165,6 +165,9 @@ int32_t tpamd_abi_version(void);
 /* Opens a context on HIP device `device` (its own default-priority stream). */
 int32_t tpamd_init(int32_t device, tpamd_ctx** out);
 int32_t tpamd_finalize(tpamd_ctx* ctx);
+/* Gives back the device memory that the context keeps to be faster: its staging
+ * and workspace buffer, and the cell copies that solves built by themselves. */
+int32_t tpamd_trim(tpamd_ctx* ctx);
 /* Message of the last failed call on ctx (or of the last failed tpamd_init when ctx is NULL). */
 const char* tpamd_last_error(const tpamd_ctx* ctx);
 
@@ -229,8 +232,10 @@ int32_t tpamd_field_mesh(tpamd_ctx* ctx, const void* data, int32_t dtype, const 
  * 4 GiB.  Results are unchanged (same values, same blend order).  A solve
  * whose gathers repay it builds the copy by itself where it takes less than
  * 1/16 of the free memory, for this field and for the snapshots of
- * tpamd_field_time_grid, until enable = 0 is asked for once.  Batches use
- * copies that were asked for only.  enable = 0 frees the copy; a batch made
+ * tpamd_field_time_grid, until enable = 0 is asked for once (the only call
+ * that takes a time grid).  Batches use copies that were asked for only.  A
+ * copy that was not asked for goes when another allocation of the context
+ * would fail, and with tpamd_trim.  enable = 0 frees the copy; a batch made
  * while an asked-for copy was there must not run after that. */
 int32_t tpamd_field_grid_cells(tpamd_ctx* ctx, tpamd_field* f, int32_t enable);
 /* E = -u x B(x) for a uniform drift u; `B` must be the B field of the solve. */

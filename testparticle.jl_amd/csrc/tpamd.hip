@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -104,7 +105,7 @@ hipError_t tpamd::ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out)
         const hipError_t e = hipMalloc(&ctx->d_buf, bytes);
         if (e != hipSuccess) {
             ctx->d_buf = nullptr;
-            (void)hipGetLastError();                     // or the next launch would report it
+            (void)hipGetLastError();
             return e;
         }
         ctx->d_buf_bytes = bytes;
@@ -181,6 +182,69 @@ hipError_t tpamd::stage_out(tpamd_ctx* ctx, const char* dev, size_t span, const 
 }
 
 namespace {
+
+// The fields (of all contexts) whose cell copy a solve built by itself.
+// Fields may be freed by other threads than the one that solves.
+std::mutex auto_mutex;
+std::vector<tpamd_field*> auto_fields;
+
+void set_cells_auto(tpamd_field* f, bool on)
+{
+    const std::lock_guard<std::mutex> lock(auto_mutex);
+    if (f->cells_auto == on) return;
+    f->cells_auto = on;
+    if (on) auto_fields.push_back(f);
+    else auto_fields.erase(std::find(auto_fields.begin(), auto_fields.end(), f));
+}
+
+// Gives back what the context holds on its own account: the cell copies that
+// solves built by themselves and, with `buffer`, its device buffer.  For use
+// between calls, or within one before it has taken a field's addresses.
+// False if there was nothing.
+bool relieve(tpamd_ctx* ctx, bool buffer)
+{
+    bool any = false;
+    {
+        const std::lock_guard<std::mutex> lock(auto_mutex);
+        auto keep = auto_fields.begin();
+        for (tpamd_field* f : auto_fields) {
+            if (f->owner != ctx) {
+                *keep++ = f;
+                continue;
+            }
+            (void)hipFree(f->cells_data);
+            f->cells_data = nullptr;
+            f->d.cells = nullptr;
+            f->cells_auto = false;
+            any = true;
+        }
+        auto_fields.erase(keep, auto_fields.end());
+    }
+    if (buffer && ctx->d_buf) {
+        (void)hipFree(ctx->d_buf);
+        ctx->d_buf = nullptr;
+        ctx->d_buf_bytes = 0;
+        any = true;
+    }
+    return any;
+}
+
+// hipMalloc for what a caller asked for: where memory has run out, what the
+// context holds on its own account goes first
+hipError_t dev_alloc(tpamd_ctx* ctx, void** out, size_t bytes, bool buffer)
+{
+    hipError_t e = hipMalloc(out, bytes);
+    if (e == hipErrorOutOfMemory && relieve(ctx, buffer)) e = hipMalloc(out, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();        // or the next launch would report it
+    return e;
+}
+
+hipError_t call_buffer(tpamd_ctx* ctx, size_t bytes, void** out)
+{
+    hipError_t e = ctx_buffer(ctx, bytes, out);
+    if (e == hipErrorOutOfMemory && relieve(ctx, false)) e = ctx_buffer(ctx, bytes, out);
+    return e;
+}
 
 // the context's pinned word for a step count read back behind a launch
 unsigned long long* pin_word(const tpamd_ctx* ctx) { return (unsigned long long*)(ctx->h_pin + kPinSlots * kPinPiece); }
@@ -417,7 +481,7 @@ double cells_bytes(const DevField& f)
 
 // builds the cell-replicated copy of a grid, or of every snapshot of a
 // sequence, by work on st
-int build_cells(tpamd_ctx* ctx, tpamd_field* f, hipStream_t st)
+int build_cells(tpamd_ctx* ctx, tpamd_field* f, hipStream_t st, bool asked)
 {
     DevField& d = f->d;
     const bool per = d.extrap == kExtrapPeriodic, f32 = d.dtype == 1;
@@ -428,7 +492,8 @@ int build_cells(tpamd_ctx* ctx, tpamd_field* f, hipStream_t st)
     const long long ncell = (long long)nc[0] * nc[1] * nc[2];
     const size_t one = ((size_t)ncell * stride + 255) / 256 * 256;
     char* cells = nullptr;
-    HIP_TRY(ctx, hipMalloc((void**)&cells, one * (size_t)snaps));
+    HIP_TRY(ctx, asked ? dev_alloc(ctx, (void**)&cells, one * (size_t)snaps, true)
+                       : hipMalloc((void**)&cells, one * (size_t)snaps));
     const unsigned blocks = (unsigned)((ncell + 255) / 256);
     for (int s = 0; s < snaps; ++s) {
         const char* nodes = (const char*)d.data + (size_t)s * (size_t)d.snap_bytes;
@@ -478,8 +543,8 @@ void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, hipStrea
         (void)hipGetLastError();
         return;
     }
-    if (build_cells(ctx, f, st) == TPAMD_OK) {
-        f->cells_auto = true;
+    if (build_cells(ctx, f, st, false) == TPAMD_OK) {
+        set_cells_auto(f, true);
     } else {                                                      // solves from the nodes then
         (void)hipGetLastError();
         ctx->err.clear();
@@ -765,7 +830,7 @@ int batch_chunks(tpamd_batch* b, int ppt, int stride)
         if (b->d_chunks) HIP_TRY(ctx, hipFree(b->d_chunks));
         b->d_chunks = nullptr;
         b->chunks_cap = 0;
-        HIP_TRY(ctx, hipMalloc((void**)&b->d_chunks, sizeof(Chunk) * std::max<size_t>(ch.size(), 1)));
+        HIP_TRY(ctx, dev_alloc(ctx, (void**)&b->d_chunks, sizeof(Chunk) * std::max<size_t>(ch.size(), 1), false));
         b->chunks_cap = ch.size();
     }
     if (!ch.empty())
@@ -946,6 +1011,7 @@ static int32_t new_field(tpamd_ctx* ctx, tpamd_field** out, int kind)
     f->cells_data = nullptr;
     f->cells_off = false;
     f->cells_auto = false;
+    f->owner = ctx;
     f->src = nullptr;
     f->bytes = 0;
     *out = f;
@@ -1056,7 +1122,7 @@ int32_t tpamd_field_grid(tpamd_ctx* ctx, const void* data, int32_t dtype, int64_
     const size_t es = storage_dtype == TPAMD_F64 ? 8 : 4;
     void* dev = nullptr;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMalloc(&dev, nn * es));
+    HIP_TRY(ctx, dev_alloc(ctx, &dev, nn * es, true));
     const hipError_t e = upload_nodes(dev, data, dtype, nn, storage_dtype);
     if (e != hipSuccess) {
         (void)hipFree(dev);
@@ -1100,7 +1166,7 @@ int32_t tpamd_field_time_grid(tpamd_ctx* ctx, const void* const* snapshots, int3
     const size_t snap = (nn * es + 255) / 256 * 256;
     void* dev = nullptr;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMalloc(&dev, head + snap * (size_t)nsnap));
+    HIP_TRY(ctx, dev_alloc(ctx, &dev, head + snap * (size_t)nsnap, true));
     hipError_t e = hipMemcpy(dev, times, (size_t)nsnap * 8, hipMemcpyHostToDevice);
     for (int k = 0; e == hipSuccess && k < nsnap; ++k)
         e = upload_nodes((char*)dev + head + (size_t)k * snap, snapshots[k], dtype, nn, storage_dtype);
@@ -1229,7 +1295,7 @@ int32_t tpamd_field_mesh(tpamd_ctx* ctx, const void* data, int32_t dtype, const 
     const size_t total = off_data + nn * es;
     char* dev = nullptr;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
-    HIP_TRY(ctx, hipMalloc((void**)&dev, total));
+    HIP_TRY(ctx, dev_alloc(ctx, (void**)&dev, total, true));
     hipError_t e = hipSuccess;
     for (int d = 0; d < 3 && e == hipSuccess; ++d) {
         g.ax[d].c = (const double*)(dev + off_c[d]);
@@ -1277,6 +1343,7 @@ int32_t tpamd_field_free(tpamd_ctx* ctx, tpamd_field* f)
 {
     if (!f) return TPAMD_OK;
     if (ctx) (void)hipSetDevice(ctx->device);
+    set_cells_auto(f, false);
     if (f->dev_data) (void)hipFree(f->dev_data);
     if (f->cells_data) (void)hipFree(f->cells_data);
     delete f;
@@ -1286,25 +1353,33 @@ int32_t tpamd_field_free(tpamd_ctx* ctx, tpamd_field* f)
 int32_t tpamd_field_grid_cells(tpamd_ctx* ctx, tpamd_field* f, int32_t enable)
 {
     if (!ctx || !f) return fail(ctx, TPAMD_ERR_ARGUMENT, "null argument");
-    if (f->d.kind != kFieldGrid)
+    if (f->d.kind != kFieldGrid && (enable || f->d.kind != kFieldTimeGrid))
         return fail(ctx, TPAMD_ERR_ARGUMENT, "the cell layout needs a static gridded field");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     if (!enable) {
         f->cells_off = true;
         f->d.cells = nullptr;
-        f->cells_auto = false;
+        set_cells_auto(f, false);
         if (f->cells_data) HIP_TRY(ctx, hipFree(f->cells_data));
         f->cells_data = nullptr;
         return TPAMD_OK;
     }
     f->cells_off = false;
-    f->cells_auto = false;               // the caller's from here on
+    set_cells_auto(f, false);            // the caller's from here on
     if (f->d.cells) return TPAMD_OK;
     if (cells_bytes(f->d) >= 4294967296.0)
         return fail(ctx, TPAMD_ERR_UNSUPPORTED, "cell layout needs fewer than 4 GiB of cells");
-    const int rc = build_cells(ctx, f, ctx->stream);
+    const int rc = build_cells(ctx, f, ctx->stream, true);
     if (rc) return rc;
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    return TPAMD_OK;
+}
+
+int32_t tpamd_trim(tpamd_ctx* ctx)
+{
+    if (!ctx) return fail(nullptr, TPAMD_ERR_ARGUMENT, "null context");
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    (void)relieve(ctx, true);
     return TPAMD_OK;
 }
 
@@ -1323,13 +1398,17 @@ int32_t tpamd_field_eval(tpamd_ctx* ctx, const tpamd_field* f, const tpamd_field
     std::memset(&zero, 0, sizeof zero);
     KParams p;
     std::memset(&p, 0, sizeof p);
-    int rc = uxb ? setup_fields(ctx, f, B, precision, p) : setup_fields(ctx, &zero, f, precision, p);
+    auto setup = [&] {
+        return uxb ? setup_fields(ctx, f, B, precision, p) : setup_fields(ctx, &zero, f, precision, p);
+    };
+    const int rc = setup();
     if (rc) return rc;
     const int which = uxb ? 1 : 0;
     if (n == 0) return TPAMD_OK;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     double* dx = nullptr;
-    HIP_TRY(ctx, hipMalloc((void**)&dx, sizeof(double) * 6 * n));
+    HIP_TRY(ctx, dev_alloc(ctx, (void**)&dx, sizeof(double) * 6 * n, true));
+    (void)setup();                       // the fields' copies may have gone for it
     double* dout = dx + 3 * n;
     hipError_t e = hipMemcpyAsync(dx, x, sizeof(double) * 3 * n, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) {
@@ -1365,7 +1444,9 @@ int32_t tpamd_record_eval(tpamd_ctx* ctx, const tpamd_field* E, const tpamd_fiel
     const int w = p.rec_w - 6;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     double* dxv = nullptr;
-    HIP_TRY(ctx, hipMalloc((void**)&dxv, sizeof(double) * (7 + (size_t)w) * n));
+    HIP_TRY(ctx, dev_alloc(ctx, (void**)&dxv, sizeof(double) * (7 + (size_t)w) * n, true));
+    p.B = B->d;                          // the fields' copies may have gone for it
+    p.E = E->d;
     double* dt = dxv + 6 * n;
     double* dout = dt + n;
     hipError_t e = hipMemcpyAsync(dxv, xv, sizeof(double) * 6 * n, hipMemcpyHostToDevice, ctx->stream);
@@ -1440,7 +1521,7 @@ int32_t tpamd_solve(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fi
                  o_t = o_u + al(b_u), o_len = o_t + al(b_t), o_ret = o_len + al(b_i), need = o_ret + al(b_i);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     char* d = nullptr;
-    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&d));
+    HIP_TRY(ctx, call_buffer(ctx, need, (void**)&d));
     hipStream_t st = ctx->stream;
     unsigned long long steps = 0;
     Drain drain{st};
@@ -1532,7 +1613,11 @@ int32_t tpamd_adjoint(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_
     rc = launch(ckpt);
     // free memory is a figure of the moment (other processes, and what one
     // allocation may take at most): the call needs no more than its checkpoints
-    if (rc == TPAMD_ERR_OOM && !ckpt) rc = launch(true);
+    // and the nodes
+    if (rc == TPAMD_ERR_OOM && (relieve(ctx, true) || !ckpt)) {
+        p.B = B->d;
+        rc = launch(true);
+    }
     drain.done = rc == TPAMD_OK;
     return rc;
 }
@@ -1584,7 +1669,9 @@ int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpa
     const size_t need = al(b_st) + al(b_it) + 2 * al(b_i) + al(b_sy) + al(b_u) + al(b_t);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     char* b = nullptr;
-    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&b));
+    HIP_TRY(ctx, call_buffer(ctx, need, (void**)&b));
+    p.B = B->d;                          // the fields' copies may have gone for it
+    p.E = E->d;
     FoArgs a;
     a.state = (double*)b; b += al(b_st);
     a.iters = (long long*)b; b += al(b_it);
@@ -1710,10 +1797,10 @@ int32_t tpamd_batch_create(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t
     hipDeviceProp_t prop;
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess) e = hipGetDeviceProperties(&prop, ctx->device);
-    if (e == hipSuccess) e = hipMalloc((void**)&b->d_table, sizeof(KParams) * n_inst);
+    if (e == hipSuccess) e = dev_alloc(ctx, (void**)&b->d_table, sizeof(KParams) * n_inst, false);
     // kQueues claim counters 128 B apart, then the step counter
     const size_t ctr_bytes = sizeof(unsigned) * kQueues * kQueueStride;
-    if (e == hipSuccess) e = hipMalloc((void**)&b->d_counter, ctr_bytes + 128);
+    if (e == hipSuccess) e = dev_alloc(ctx, (void**)&b->d_counter, ctr_bytes + 128, false);
     if (e == hipSuccess)
         e = hipMemcpy(b->d_table, b->table.data(), sizeof(KParams) * n_inst, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
@@ -1899,7 +1986,7 @@ int32_t tpamd_solve_batch(tpamd_ctx* ctx, const tpamd_solve_desc* desc, int32_t 
     const size_t need = al(b_xv) + al(b_u) + al(b_t) + 2 * al(b_i);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     char* p = nullptr;
-    HIP_TRY(ctx, ctx_buffer(ctx, need, (void**)&p));
+    HIP_TRY(ctx, call_buffer(ctx, need, (void**)&p));
     double* d_xv = (double*)p; p += al(b_xv);
     double* d_u = (double*)p; p += al(b_u);
     double* d_t = (double*)p; p += al(b_t);

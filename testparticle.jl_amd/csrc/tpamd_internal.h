@@ -17,7 +17,9 @@ struct tpamd_field {
     void* dev_data;          // owned device buffer (grids)
     void* cells_data;        // owned cell-replicated copy (grids, optional)
     bool cells_off;          // the caller dropped the copy: no solve builds it again
-    bool cells_auto;         // a solve built it and the caller has not asked for it: no batch uses it
+    bool cells_auto;         // a solve built it and the caller has not asked for it: no batch uses it,
+                             // and it may go between calls (relieve)
+    tpamd_ctx* owner;        // the context whose calls use the field
     const tpamd_field* src;  // UxB: the B field it was built from
     size_t bytes;
     tpamd::MeshGrid mesh_host;      // Mesh: host copy of the descriptor (device pointers)
@@ -57,6 +59,7 @@ hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsig
 
 // The context's device buffer, grown to `bytes` (contents are lost): for use
 // within one call, which the caller serialises and which ends synchronised.
+// A failure leaves no buffer and no error for the next launch to report.
 hipError_t ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out);
 // releases it when it has grown past what is kept between calls
 constexpr size_t kKeepBytes = (size_t)4 << 30;

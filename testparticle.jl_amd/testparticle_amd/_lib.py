@@ -77,7 +77,7 @@ class Stats(C.Structure):
 
 
 EXPORTS = [
-    "tpamd_abi_version", "tpamd_init", "tpamd_finalize", "tpamd_last_error",
+    "tpamd_abi_version", "tpamd_init", "tpamd_finalize", "tpamd_trim", "tpamd_last_error",
     "tpamd_field_zero", "tpamd_field_uniform", "tpamd_field_affine", "tpamd_field_dipole",
     "tpamd_field_grid", "tpamd_field_time_grid", "tpamd_field_mesh", "tpamd_field_grid_cells",
     "tpamd_field_uxb",
@@ -214,6 +214,11 @@ class Context:
         if rc == ERR_NONFINITE:
             raise FloatingPointError(msg)
         raise DeviceError(msg)
+
+    def trim(self):
+        """Gives back the device memory kept between calls (tpamd_trim)."""
+        with self.lock:
+            self.check(self.L.tpamd_trim(self.h))
 
     def close(self):
         if self.h:

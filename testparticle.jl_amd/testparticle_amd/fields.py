@@ -172,12 +172,14 @@ class GridField(AbstractField):
     one block: one cache line per gather for float storage, ~10x the memory)
     when the field is created; with `layout="nodes"` the first solve with
     enough gathers to repay it does, if the copy takes less than 1/16 of the
-    free device memory.  Results are identical."""
+    free device memory; with `layout="nodes_only"` none does (the first
+    snapshot's layout is that of a LazyTimeInterpolator).  Results are
+    identical."""
 
     def __init__(self, A, x, y, z, bc=None, storage=None, layout="nodes"):
         super().__init__()
-        if layout not in ("nodes", "cells"):
-            raise _lib.ArgumentError("layout must be 'nodes' or 'cells'")
+        if layout not in ("nodes", "cells", "nodes_only"):
+            raise _lib.ArgumentError("layout must be 'nodes', 'cells' or 'nodes_only'")
         self.layout = layout
         A = np.asarray(A)
         if A.ndim != 4 or A.shape[0] != 3:
@@ -212,8 +214,8 @@ class GridField(AbstractField):
         rc = ctx.L.tpamd_field_grid(ctx.h, self.data.ctypes.data, dt, *self.shape,
                                     _lib.dptr(self.origin), _lib.dptr(self.spacing),
                                     self.extrap, st, C.byref(h))
-        if rc == _lib.OK and self.layout == "cells":
-            rc = ctx.L.tpamd_field_grid_cells(ctx.h, h, 1)
+        if rc == _lib.OK and self.layout != "nodes":
+            rc = ctx.L.tpamd_field_grid_cells(ctx.h, h, int(self.layout == "cells"))
             if rc != _lib.OK:
                 msg = ctx.L.tpamd_last_error(ctx.h)
                 ctx.L.tpamd_field_free(ctx.h, h)
@@ -286,9 +288,12 @@ class LazyTimeInterpolator(AbstractField):
         ptrs = (C.c_void_p * len(datas))(*[d.ctypes.data for d in datas])
         dt = _lib.F64 if datas[0].dtype == np.float64 else _lib.F32
         st = _lib.F64 if self.storage == "f64" else _lib.F32
-        return ctx.L.tpamd_field_time_grid(ctx.h, ptrs, dt, *self.shape, len(datas),
-                                           _lib.dptr(self.times), _lib.dptr(self.origin),
-                                           _lib.dptr(self.spacing), self.extrap, st, C.byref(h))
+        rc = ctx.L.tpamd_field_time_grid(ctx.h, ptrs, dt, *self.shape, len(datas),
+                                         _lib.dptr(self.times), _lib.dptr(self.origin),
+                                         _lib.dptr(self.spacing), self.extrap, st, C.byref(h))
+        if rc == _lib.OK and self._first.layout == "nodes_only":
+            rc = ctx.L.tpamd_field_grid_cells(ctx.h, h, 0)
+        return rc
 
 
 class UxBField(AbstractField):
