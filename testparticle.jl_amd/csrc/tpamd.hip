@@ -448,12 +448,19 @@ void select_policy(const tpamd_solve_desc* d, const KParams& p, bool allow_spec,
     const bool special = !(d->flags & TPAMD_FLAG_GENERIC_KERNELS);
     // two gathers a step: gridded E and B on one geometry (both with cells or
     // both without), or B a sequence of snapshots (fixed-step Boris, plain
-    // records, node arrays that 32-bit offsets reach)
+    // records, node arrays that 32-bit offsets reach).  Float nodes at FP32C
+    // are the exception: with a wave on every SIMD the generic kernels are the
+    // faster ones (100,000 particles, E and B of 28^3 1.4 times, of 80^3 1.15;
+    // 200,000, snapshots of 56^3 1.09), for E and B beyond 4 MiB of L2 always
+    // (500 particles, 80^3: 1.05); elsewhere the pair is (50,000 particles,
+    // snapshots of 28^3: 1.7 times)
     const bool flat = p.e_is_uxb || p.E.kind == kFieldZero || p.E.kind == kFieldUniform;
     const bool time = p.B.kind == kFieldTimeGrid && flat;
     const bool eb = p.B.kind == kFieldGrid && !p.e_is_uxb && p.E.kind == kFieldGrid && p.E.dtype == p.B.dtype &&
                     (p.E.cells != nullptr) == (p.B.cells != nullptr) && same_geometry(p.E, p.B);
-    if (special && !r.batch && !r.adaptive && p.alg == TPAMD_ALG_BORIS && p.rec_w == 6 && (time || eb) &&
+    const bool nodes32 = d->precision == TPAMD_FP32C && !p.B.cells &&
+                         (p.N >= 65536 || (eb && 2.0 * nodes_bytes(p.B) > 4.0 * 1048576.0));
+    if (special && !r.batch && !r.adaptive && p.alg == TPAMD_ALG_BORIS && p.rec_w == 6 && (time || eb) && !nodes32 &&
         nodes_bytes(p.B) < 4294967296.0 && (d->precision == TPAMD_FP64 || p.B.dtype == 1)) {
         const bool per = p.B.extrap == kExtrapPeriodic, cells = p.B.cells != nullptr;
         if (d->precision == TPAMD_FP32C) launch_pair32(r, time, p.e_is_uxb != 0, per, cells);
@@ -519,27 +526,65 @@ int build_cells(tpamd_ctx* ctx, tpamd_field* f, hipStream_t st, bool asked)
     return TPAMD_OK;
 }
 
+// Nanoseconds that a gather of one array saves on cells, 0 where it saves none
+// (E: a gridded E, or null).  Measured on cubes of 16 to 192 nodes an edge, 500
+// to 400,000 particles, nodes against cells, per particle-step:
+//   * Node arrays beyond one XCD's 4 MiB of L2: always faster, 1.2-5 times.
+//     400,000 particles save 0.027-0.046 ns a gather below some 16 MiB and
+//     0.045-0.09 above (random lines), few particles a step's latency, 1.0 us
+//     (float) and 1.8-1.9 (double; 64^3, 500 particles: 6.2 -> 2.7 ns, 400,000:
+//     0.076 -> 0.040).
+//   * Within it, the nodes' 4 to 8 lines come from the L2 and the cells, 8-10
+//     times as large, do not.  Up to 50,000 particles cells are slower, 0.79 to
+//     1.0 times; with a wave and more on every SIMD their fewer requests win,
+//     1.2-2.0 times (48^3 double, 20,000 particles: 0.90 times, 100,000: 1.20;
+//     float 0.89 and 2.02).  Two doubles a step turn later (snapshots of 32^3,
+//     100,000: 0.78 times, 200,000: 1.16), or not at all (E and B of 32^3,
+//     400,000: 0.89); float E and B win throughout (1.05-2.1 times).  Where the
+//     cells fit as well (up to 0.5 MiB of nodes), double ones are 1.2-1.45 times
+//     faster at any number (16^3, 500 particles: 2.53 -> 2.11 ns), float ones
+//     0.88-1.0.
+//   * The gradient, whose reverse sweep reads a cell's 24 values as they lie:
+//     never slower within it, 1.1-1.46 times for double (48^3, 5,000 particles),
+//     1.0-1.2 for float; beyond it as above.
+double cells_gain(const DevField& B, const DevField* E, long long N, bool gradient)
+{
+    auto lone = [](const DevField& f) { return is_gridded(f) ? nodes_bytes(f) * (f.nsnap > 1 ? 2.0 : 1.0) : 0.0; };
+    const bool both = E && is_gridded(B);
+    const DevField& f = is_gridded(B) ? B : *E;
+    const double mib = (lone(B) + (E ? lone(*E) : 0.0)) / 1048576.0;
+    if (mib > 4.0)
+        return std::max(mib > 16.0 ? 0.045 : 0.028, (f.dtype == 1 ? 1000.0 : 1800.0) / (double)std::max(N, 1LL));
+    if (gradient) return f.dtype == 1 ? 0.002 : std::max(0.006, 360.0 / (double)N);
+    if (f.dtype != 1 && mib <= 0.5) return std::max(N >= 65536 ? 0.015 : 0.004, 200.0 / (double)std::max(N, 1LL));
+    if (both) return f.dtype == 1 ? 0.015 : 0.0;
+    return N >= (f.nsnap > 1 && f.dtype != 1 ? 131072 : 65536) ? 0.018 : 0.0;
+}
+
 // A solve of `gathers` field evaluations from a field's node array builds the
 // cell-replicated copy first, on its stream, where that repays itself within
-// the solve, and the field keeps it.  The copy counts as built at once: the
-// caller has checked its arguments, and leaves, also with an error, only when
-// the stream has been waited for (Drain), so that the next solve finds it on
-// any stream.  Measured over grids from 2 MB to 3 GB: a
-// gather from double nodes reads 4-8 random lines, 1.0-1.6e10 gathers/s, one
-// from cells two, 2.8-6.5e10 (float: 1.2e10 and 5.5-9.9e10); building writes a
-// cell in 0.05 ns, allocating takes some 15 us below 64 MB and 0.05-0.4 ms
-// above.  So the copy saves ~0.06 ns a gather and has paid from one gather per
-// cell plus some 8e5 on.  It takes at most 1/16 of the free memory, and a
-// caller that dropped a field's copy gets none.
-void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, hipStream_t st)
+// the solve, and the field keeps it.  Building takes some 50 us and 0.45 us a
+// MB of cells, and 120 us more to allocate above 64 MB (6 MB 49 us, 50 MB 62,
+// 113 MB 200-275, 170 MB 195-260, 403 MB 280-330, 1.36 GB 720-850; the
+// first of a size in a process up to 0.5 ms).  The gathers are those of a solve
+// whose particles all live to its end: lives that a boundary ends in the first
+// steps build a copy for nothing, once a field (100,000 particles gone within
+// two of 1,000 steps, 128^3: 0.20 -> 0.6 ms).  A copy takes at most 1/16 of the
+// free memory, and a caller that dropped a field's copy gets none.  The copy
+// counts as built at once: the caller has checked its arguments, and leaves,
+// also with an error, only when the stream has been waited for (Drain), so
+// that the next solve finds it on any stream.
+void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, double gain, hipStream_t st)
 {
     tpamd_field* f = const_cast<tpamd_field*>(cf);
-    const int snaps = f->d.kind == kFieldTimeGrid ? f->d.nsnap : 1;
-    if ((f->d.kind != kFieldGrid && f->d.kind != kFieldTimeGrid) || f->d.cells || f->cells_off) return;
-    const double bytes = cells_bytes(f->d), ncell = bytes / (f->d.dtype == 1 ? 128.0 : 192.0) * snaps;
-    if (bytes >= 4294967296.0 || gathers < ncell + 8.0e5) return;
+    if (!is_gridded(f->d) || f->d.cells || f->cells_off) return;
+    const bool time = f->d.kind == kFieldTimeGrid;
+    const double one = cells_bytes(f->d), all = one * (time ? f->d.nsnap : 1);
+    if (f->d.nsnap > 1) gathers *= 2.0;                           // blends two snapshots
+    if (one >= 4294967296.0 || gathers * gain < 5.0e4 + 4.5e-4 * all + (all > 6.4e7 ? 1.2e5 : 0.0))
+        return;
     size_t mem_free = 0, mem_total = 0;
-    if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess || bytes * snaps > (double)mem_free / 16.0) {
+    if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess || all > (double)mem_free / 16.0) {
         (void)hipGetLastError();
         return;
     }
@@ -549,6 +594,25 @@ void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, hipStrea
         (void)hipGetLastError();
         ctx->err.clear();
     }
+}
+
+// The fields of a solve of N particles and `gathers` evaluations as its
+// kernels see them: with cells where that is faster, or where the caller asked
+// for a copy.  (The results are the same bits.)
+void settle_cells(tpamd_ctx* ctx, const tpamd_field* E, const tpamd_field* B, long long N, double gathers,
+                  hipStream_t st, KParams& p, bool gradient = false)
+{
+    const bool e = !p.e_is_uxb && is_gridded(E->d);
+    if (!e && !is_gridded(B->d)) return;
+    const double gain = cells_gain(B->d, e ? &E->d : nullptr, N, gradient);
+    if (gain > 0.0) {
+        offer_cells(ctx, B, gathers, gain, st);
+        if (e) offer_cells(ctx, E, gathers, gain, st);
+    }
+    p.B = B->d;
+    p.E = E->d;
+    const bool asked = (B->d.cells && !B->cells_auto) || (e && E->d.cells && !E->cells_auto);
+    if (gain <= 0.0 && !asked) p.B.cells = p.E.cells = nullptr;
 }
 
 // Validates the descriptor and fills the kernel parameter block (everything
@@ -697,11 +761,7 @@ int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fiel
     p.span = (int)(64 * ppl);
     if (!(desc->flags & TPAMD_FLAG_GENERIC_KERNELS)) {
         // an adaptive particle's steps are not known: two evaluations at least
-        const double gathers = (double)N * (desc->adaptive ? 2.0 : (double)nt + 1.0);
-        offer_cells(ctx, B, gathers, st);
-        if (!p.e_is_uxb) offer_cells(ctx, E, gathers, st);
-        p.B = B->d;
-        p.E = E->d;
+        settle_cells(ctx, E, B, N, (double)N * (desc->adaptive ? 2.0 : (double)nt + 1.0), st, p);
     }
     if (N > 0) {
         const long long threads = desc->adaptive ? (N + p.span - 1) / p.span * 64 : N;
@@ -1600,10 +1660,9 @@ int32_t tpamd_adjoint(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_
         return fail(ctx, TPAMD_ERR_CAPACITY, "too many adjoint records: lower the checkpoint interval or N");
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     Drain drain{ctx->stream};                       // adjoint_launch leaves early where it fails
-    if (bf32 == f32) {                              // the adjoint's kernels on cells
-        offer_cells(ctx, B, 2.0 * (double)N * (double)nt, ctx->stream);
-        p.B = B->d;
-    }
+    // forward and reverse; the FP64 kernels on float nodes read no cells
+    if (bf32 == f32) settle_cells(ctx, &zero, B, N, 2.0 * (double)N * (double)nt, ctx->stream, p, true);
+    else p.B.cells = nullptr;
     auto launch = [&](bool ckpt) {
         const bool cells = p.B.cells != nullptr;    // gathers from the cell-replicated copy
         return adjoint_launch(ctx, p, B, xv0, N, targets, ckpt_interval, nt, loss, dL_dB, dL_dxv0, stats,
@@ -1670,8 +1729,7 @@ int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpa
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     char* b = nullptr;
     HIP_TRY(ctx, call_buffer(ctx, need, (void**)&b));
-    p.B = B->d;                          // the fields' copies may have gone for it
-    p.E = E->d;
+    settle_cells(ctx, E, B, N, 0.0, ctx->stream, p);     // builds none
     FoArgs a;
     a.state = (double*)b; b += al(b_st);
     a.iters = (long long*)b; b += al(b_it);

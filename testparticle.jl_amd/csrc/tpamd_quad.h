@@ -199,14 +199,15 @@ struct Out {
 };
 
 // n steps, none of which saves (boris.jl:454-457): q triples and r single
-// ones.  The triples' loop starts on a 64-B line: a lone wave's time depends
-// on where its 7-8 lines of instructions begin (1,000 particles x 3,000 steps
-// FP64, E zero: 0.119 ms, 0.126-0.128 where it fell before; E not zero 0.135,
-// 0.139-0.146).
-template <class R, class M, bool EZ>
+// ones.  ALIGN: the triples' loop starts on a 64-B line, as a lone wave's time
+// depends on where its 7-8 lines of instructions begin (1,000 particles x 3,000
+// steps FP64, E zero: 0.119 ms, 0.125-0.128 where it fell by itself; E not zero
+// 0.135, 0.139-0.146).  Not between saves, where the padding runs each time (7
+// x 500 steps, every fifth saved: 48 us with, 46 without).
+template <bool ALIGN, class R, class M, bool EZ>
 __device__ __forceinline__ void steps(const Spin<R, EZ>& step, R& v, M& m, int q, int r)
 {
-    asm volatile(".p2align 6");
+    if constexpr (ALIGN) asm volatile(".p2align 6");
     for (; q > 0; --q) {
         R vc;
         m.clock();
@@ -261,8 +262,8 @@ __device__ __forceinline__ void run(const KParams& p, long long i, int lc, const
     long long quiet = p.save_every && p.K < nt ? p.K : nt;    // of which none of these saves
     const long long between = p.K - 1 < nt ? p.K - 1 : nt;
     const int bq = (int)(between < kMost ? between / 3 : 0), br = (int)(between < kMost ? between % 3 : 0);
-    for (; quiet > kMost; quiet -= kMost, left -= kMost) steps<R, M, EZ>(step, v, m, 1 << 30, 0);
-    steps<R, M, EZ>(step, v, m, (int)(quiet / 3), (int)(quiet % 3));
+    for (; quiet > kMost; quiet -= kMost, left -= kMost) steps<true, R, M, EZ>(step, v, m, 1 << 30, 0);
+    steps<true, R, M, EZ>(step, v, m, (int)(quiet / 3), (int)(quiet % 3));
     left -= quiet;
     while (left > 0) {
         const R vprev = v;                                    // a step that saves (:463-472)
@@ -277,13 +278,13 @@ __device__ __forceinline__ void run(const KParams& p, long long i, int lc, const
         }
         left -= 1;
         if (left >= between && between < kMost) {
-            steps<R, M, EZ>(step, v, m, bq, br);
+            steps<false, R, M, EZ>(step, v, m, bq, br);
             left -= between;
         } else {
             quiet = left < between ? left : between;
             left -= quiet;
-            for (; quiet > kMost; quiet -= kMost) steps<R, M, EZ>(step, v, m, 1 << 30, 0);
-            steps<R, M, EZ>(step, v, m, (int)(quiet / 3), (int)(quiet % 3));
+            for (; quiet > kMost; quiet -= kMost) steps<false, R, M, EZ>(step, v, m, 1 << 30, 0);
+            steps<false, R, M, EZ>(step, v, m, (int)(quiet / 3), (int)(quiet % 3));
         }
     }
     // no particle leaves: every one makes nt steps

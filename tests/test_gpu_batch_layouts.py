@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["fp64", "fp32c"])
 def test_batch_after_a_solve_of_one_field(precision, layouts):
     rng = np.random.default_rng(11)
-    L, m, n, nt = 1.0e8, 14, 9001, 100               # n * nt gathers: a solve builds a copy
+    L, m, n, nt = 1.0e8, 14, 70001, 100              # n * nt gathers: a solve builds a copy
     dtype = np.float32 if precision == "fp32c" else np.float64
     q2m = TP.qi / TP.mi
 

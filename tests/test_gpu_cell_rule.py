@@ -1,0 +1,94 @@
+"""When a solve builds a cell copy by itself and when it uses one: where cells
+are faster and repay the building.  Whatever it takes, the bits are those of
+the nodes, of an asked-for copy and, for two gathers a step, of the generic
+kernels."""
+import numpy as np
+import pytest
+
+import testparticle_amd as TP
+from testparticle_amd.device import DeviceEnsemble
+
+pytestmark = pytest.mark.gpu
+
+L, Q2M = 1.0e8, TP.qi / TP.mi
+BCS = {"periodic": TP.PeriodicBC, "clamp": TP.ClampExtrap, "fill": TP.FillExtrap}
+
+
+def grid(shape, seed, bc, dtype, layout, scale=1e-9, mean=5e-9):
+    A = np.random.default_rng(seed).normal(0.0, scale, (3,) + shape)
+    A[2] += mean
+    ax = [np.arange(n) * (L / n if bc == "periodic" else L / (n - 1)) for n in shape]
+    return TP.GridField(A.astype(dtype), *ax, bc=BCS[bc](), layout=layout)
+
+
+def fields(kind, shape, bc, dtype, layout):
+    """A gridded B, E and B, or three snapshots of B."""
+    if kind == "one":
+        return TP.UniformField([0.0, 5e-4, 0.0]), grid(shape, 1, bc, dtype, layout)
+    if kind == "pair":
+        return grid(shape, 2, bc, dtype, layout, 1e-3, 5e-4), grid(shape, 1, bc, dtype, layout)
+    return TP.ZeroField(), TP.LazyTimeInterpolator([0.0, 2.0, 9.0], lambda i: grid(shape, i, bc, dtype, layout))
+
+
+def particles(n):
+    rng = np.random.default_rng(n)
+    return np.hstack([rng.uniform(0.1 * L, 0.9 * L, (n, 3)), rng.normal(0.0, 1.5e6, (n, 3))])
+
+
+# below and above the particles from which small grids pay, with steps that
+# repay the copy where it does
+@pytest.mark.parametrize("bc", list(BCS))
+@pytest.mark.parametrize("precision,dtype", [("fp64", np.float64), ("fp64", np.float32), ("fp32c", np.float32)])
+@pytest.mark.parametrize("kind", ["one", "pair", "time"])
+@pytest.mark.parametrize("n,nt", [(1, 3), (65, 40), (9001, 20), (65535, 90), (65537, 90), (131073, 40)])
+def test_every_route_gives_the_same_bits(kind, precision, dtype, bc, n, nt):
+    xv = particles(n)
+    kw = dict(dt=0.3, precision=precision, save_everystep=False, isoutside=None if bc == "periodic" else TP.OutsideGrid())
+
+    def run(layout, **more):
+        E, B = fields(kind, (9, 7, 11), bc, dtype, layout)
+        e = DeviceEnsemble(TP.TraceProblem(xv, (0.0, nt * 0.3), (Q2M, TP.mi, E, B, TP.ZeroField())), TP.Boris(), xv,
+                           **kw, **more)
+        out = []
+        for _ in range(2):
+            for a in (e.u, e.t, e.len, e.ret):
+                a.zero_()
+            e.run()
+            out.append([a.cpu().numpy() for a in (e.u, e.t, e.len, e.ret)])
+        return out
+
+    want = run("nodes_only")
+    others = [run("nodes"), run("cells")] + ([run("nodes_only", kernels="generic")] if kind != "one" else [])
+    for got in [want[1]] + [g for o in others for g in o]:
+        for a, b in zip(got, want[0]):
+            np.testing.assert_array_equal(a.view(np.int32), b.view(np.int32))
+
+
+def taken(kind, m, dtype, n, nt):
+    """Device memory that a first solve leaves taken."""
+    import torch
+    E, B = fields(kind, (m, m, m), "periodic", dtype, "nodes")
+    xv = particles(n)
+    e = DeviceEnsemble(TP.TraceProblem(xv, (0.0, nt * 0.3), (Q2M, TP.mi, E, B, TP.ZeroField())), TP.Boris(), xv, dt=0.3,
+                       save_everystep=False, precision="fp32c" if dtype == np.float32 else "fp64")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    e.run()
+    torch.cuda.synchronize()
+    return before - torch.cuda.mem_get_info()[0]
+
+
+# (kind, nodes an edge, type, particles, steps) and whether a copy is built
+@pytest.mark.parametrize("case,built", [
+    (("one", 48, np.float64, 20000, 1500), False),      # 2.7 MB of nodes: the L2 holds them
+    (("one", 48, np.float64, 65536, 100), True),
+    (("one", 64, np.float32, 20000, 1500), False),
+    (("one", 64, np.float64, 2000, 300), True),         # 6.3 MB: it does not
+    (("one", 64, np.float64, 2000, 20), False),         # too few steps to repay it
+    (("one", 64, np.float64, 200000, 2), False),
+    (("pair", 32, np.float64, 200000, 60), False),
+    (("time", 40, np.float64, 70000, 200), False),
+    (("time", 40, np.float64, 140000, 200), True),
+])
+def test_when_a_copy_is_built(case, built):
+    assert (taken(*case) > 8 << 20) == built
