@@ -53,8 +53,9 @@ GATHER_BYTES = {"f32": 8 * 3 * 4, "f64": 8 * 3 * 8}
 # return code (2 x int32) written; per record: x, v (6 doubles) and t
 STATE_BYTES, LEN_BYTES, RECORD_BYTES = 6 * 8, 2 * 4, 7 * 8
 # adjoint: a trajectory row (cell, weights, velocity), written by the forward
-# pass; the reverse sweep per particle-step reads it, gathers, and has a dL/dB
-# record (key + Bbar + weights) written and read
+# pass (or, with checkpoints, by a second gather in the reverse sweep); the
+# reverse sweep per particle-step reads it, gathers, and has a dL/dB record
+# (key + Bbar + weights) written and read
 ADJ_ROW_BYTES = {"fp32c": 4 + 6 * 4, "fp64": 4 + 6 * 8}
 ADJ_REVERSE_BYTES = {"fp32c": 96 + ADJ_ROW_BYTES["fp32c"] + 2 * 32, "fp64": 192 + ADJ_ROW_BYTES["fp64"] + 2 * 52}
 # algorithmic FLOPs per particle-step (FMA = 2; div, sqrt = 1): standard Boris
@@ -597,7 +598,10 @@ def bench_adjoint(args, torch, TP, W, DeviceEnsemble):
     tg = rng.uniform(0, L, size=(N, 3))
     dt = 2 * math.pi * TP.mi / (TP.qi * B0) / 40
     q2m = TP.qi / TP.mi
-    log(f"[bench] adjoint: {n}^3 grid, {N} protons x {nsteps} steps, checkpoints every {K}")
+    # a trajectory of up to 1/16 of the memory is kept whole (the library's own choice)
+    whole = {p: N * (nsteps + 1) * ADJ_ROW_BYTES[p] < torch.cuda.mem_get_info()[1] / 17 for p in ADJ_ROW_BYTES}
+    log(f"[bench] adjoint: {n}^3 grid, {N} protons x {nsteps} steps, "
+        + ", ".join(f"{p} {'whole trajectory' if w else f'checkpoints every {K}'}" for p, w in whole.items()))
 
     def prob_of(Av, storage, h=nsteps, layout="cells"):
         B = TP.GridField(Av, *ax, bc=TP.PeriodicBC(), storage=storage, layout=layout)
@@ -605,7 +609,8 @@ def bench_adjoint(args, torch, TP, W, DeviceEnsemble):
 
     def grad(prec, h):
         storage = "f32" if prec == "fp32c" else "f64"
-        return TP.loss_gradient(prob_of(A, storage, h), dt=dt, targets=tg, precision=prec, ckpt_interval=K)
+        return TP.loss_gradient(prob_of(A, storage, h), dt=dt, targets=tg, precision=prec, ckpt_interval=K,
+                                checkpoints=h == nsteps and not whole[prec])
 
     out = {"workload": "adjoint_turbulent_64^3", "particles": N, "steps": nsteps,
            "checkpoint_interval": K, "dt": "T_g(B0)/40", "box": "1e7 m periodic",
@@ -640,19 +645,22 @@ def bench_adjoint(args, torch, TP, W, DeviceEnsemble):
         best = min(fwd.values())
         g = rs[-1]
         # the reverse sweep's roofline: per particle-step a row, a gather, and
-        # the dL/dB record written and read
-        abytes = ADJ_REVERSE_BYTES[prec]
+        # the dL/dB record written and read (with checkpoints a gather and a row
+        # more, and the forward pass writes no rows)
+        gather = GATHER_BYTES["f32" if prec == "fp32c" else "f64"]
+        row = ADJ_ROW_BYTES[prec]
+        abytes = ADJ_REVERSE_BYTES[prec] + (0 if whole[prec] else gather + row)
         psteps = N * nsteps
-        roof = {"bound": "hbm", "kernel": "reverse sweep: k_adj_reverse + k_adj_bins_seg",
+        roof = {"bound": "hbm", "kernel": "reverse sweep: " + ("" if whole[prec] else "k_adj_rows + ")
+                                          + "k_adj_reverse + k_adj_bins_seg",
                 "achieved": psteps * abytes / (r_ms * 1e-3) / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                 "frac": psteps * abytes / (r_ms * 1e-3) / HBM_PEAK,
                 "algorithmic_bytes_per_particle_step": abytes, "traffic": None,
-                "forward_frac": psteps * GATHER_BYTES["f32" if prec == "fp32c" else "f64"]
-                                / (best * 1e-3) / HBM_PEAK}
+                "forward_frac": psteps * gather / (best * 1e-3) / HBM_PEAK}
         out[prec] = {"forward_solve_ms": fwd, "adjoint_forward_ms": f_ms, "adjoint_reverse_ms": r_ms,
                      "cost_over_forward": (f_ms + r_ms) / best, "roofline": roof,
-                     "cost_floor_by_bytes": (GATHER_BYTES["f32" if prec == "fp32c" else "f64"] + ADJ_ROW_BYTES[prec]
-                                             + abytes) / GATHER_BYTES["f32" if prec == "fp32c" else "f64"],
+                     "trajectory": "whole" if whole[prec] else "checkpoints",
+                     "cost_floor_by_bytes": (gather + (row if whole[prec] else 0) + abytes) / gather,
                      "loss": g.loss,
                      "max_abs_dL_dB": float(np.max(np.abs(g.dL_dB))),
                      "max_abs_dL_dxv0": float(np.max(np.abs(g.dL_dxv0))),

@@ -288,11 +288,11 @@ int32_t tpamd_solve_device(tpamd_ctx* ctx, const tpamd_solve_desc* desc,
  * differentiates with ForwardDiff through the CPU solve (src/utility/utility.jl,
  * test/test_derivatives.jl); there is no reverse-mode counterpart.
  *   desc: alg = BORIS, adaptive = 0, precision FP64 or FP32C, no boundary.
- *   ckpt_interval K: where the trajectory takes more than 4 GiB or half of the
- *     free device memory (or with TPAMD_FLAG_CHECKPOINTS), FP64 state
+ *   ckpt_interval K: where the trajectory takes more than 1/16 of the free
+ *     device memory and 4 GiB (or with TPAMD_FLAG_CHECKPOINTS), FP64 state
  *     checkpoints every K steps stand in for it and the reverse sweep
- *     recomputes each K-step segment.  Workspace up to 4 GiB stays with the
- *     context for the next call.
+ *     recomputes each K-step segment.  Workspace up to 1/16 of the device's
+ *     memory stays with the context for the next call (tpamd_trim).
  *   targets[N][3]; dL_dB in B's node layout [nz][ny][nx][3] (with
  *     TPAMD_FLAG_GRADIENT_BY_COMPONENT as [3][nx][ny][nz]), summed in double;
  *   dL_dxv0[N][6].  stats->kernel_ms = forward pass, aux_ms = reverse.

@@ -116,7 +116,7 @@ hipError_t tpamd::ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out)
 
 void tpamd::ctx_trim(tpamd_ctx* ctx)
 {
-    if (ctx->d_buf_bytes <= kKeepBytes) return;
+    if (ctx->d_buf_bytes <= ctx->keep_bytes) return;
     (void)hipFree(ctx->d_buf);
     ctx->d_buf = nullptr;
     ctx->d_buf_bytes = 0;
@@ -1029,6 +1029,9 @@ int32_t tpamd_init(int32_t device, tpamd_ctx** out)
         delete c;
         return fail(nullptr, TPAMD_ERR_DEVICE, "HIP context set-up failed on device %d", device);
     }
+    size_t mem_free = 0, mem_total = 0;
+    if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess) (void)hipGetLastError();
+    c->keep_bytes = std::max((size_t)4 << 30, mem_total / 16);
     // this device's copy of the allocation-free entry point's scratch array
     // (with the device current); the name is a host-side stand-in, only the
     // looked-up address may reach a kernel or a copy

@@ -565,16 +565,16 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
                  b_out = al(sizeof(double) * 3 * nnodes), b_gx = al(sizeof(double) * 6 * N), b_ls = al(sizeof(double)),
                  b_xf = al(sizeof(double) * 3 * N), b_nf = al(sizeof(unsigned long long));
     const size_t fixed = b_xv + b_tg + b_st + b_se + b_G + b_out + b_gx + b_ls + b_xf + b_nf;
-    // The whole trajectory where the workspace stays within what the context
-    // keeps between calls (and half of the free memory), or takes no more than
-    // with checkpoints; then a launch walks as many rows as make about 2^24
-    // records (some 0.5 GB in float), a multiple of a pass.  Otherwise segments
-    // of K steps.  The trajectory saves the segments' second gathers: FP32C
-    // 131,072 x 1,000 steps 11.0 ms against 12.6, FP64 262,144 x 320 12.9
-    // against 14.7.  But memory that each call allocates and frees is wiped in
+    // The whole trajectory where the workspace takes at most 1/16 of the free
+    // memory (or 4 GiB, or no more than with checkpoints), which the context
+    // keeps for the next call; then a launch walks as many rows as make about
+    // 2^24 records (some 0.5 GB in float), a multiple of a pass.  Otherwise
+    // segments of K steps.  The trajectory saves the segments' second gathers:
+    // FP32C 262,144 x 2,048 steps (15 GB) 40 ms against 48, FP64 131,072 x 1,000
+    // (7 GB) 17 and 22.  But memory that each call allocates and frees is wiped in
     // between, at some 30 ms a GB once the device has been through its free
-    // memory: FP64 131,072 x 1,000 (7 GB) took 218 ms a call whole and 21.8 with
-    // checkpoints, 1 M x 2,048 FP32C (60 GB) 1,620 and 200.
+    // memory: not kept, the same FP64 call took 218 ms, 1 M x 2,048 FP32C (60 GB)
+    // 1,620 against 200.
     size_t mem_free = 0, mem_total = 0;
     HIP_TRY(ctx, hipMemGetInfo(&mem_free, &mem_total));
     mem_free += ctx->d_buf_bytes;                            // ours to use again
@@ -590,7 +590,7 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
     const int64_t rows_seg = std::min<int64_t>((int64_t)K + 1, nrows);
     const size_t need_whole = fixed + row_bytes(nrows) + rec_bytes(rows_launch),
                  need_ckpt = fixed + al(sizeof(double) * 9 * (size_t)nseg * N) + row_bytes(rows_seg) + rec_bytes(rows_seg);
-    const bool whole = !ckpt && (need_whole <= std::min(kKeepBytes, mem_free / 2) || need_whole <= need_ckpt);
+    const bool whole = !ckpt && (need_whole <= std::min(std::max((size_t)4 << 30, mem_free / 16), mem_free / 2) || need_whole <= need_ckpt);
     if (!whole) rows_launch = rows_seg;
     const size_t slots = rec_slots(rows_launch);
     int cellbits = 0;
@@ -606,7 +606,7 @@ int adjoint_run(tpamd_ctx* ctx, KParams p, const tpamd_field* B, const double* x
                  seg_words = (size_t)nbins * (slots / P),         // and the bins' totals behind them
                  b_seg = al(sort ? sizeof(unsigned) * (seg_words + nbins) : 1), b_tmp = al(std::max<size_t>(temp_bytes, 1));
     const size_t total = fixed + b_ck + b_rw + b_rk + (sort ? 1 : 2) * (b_key + b_val) + b_seg + b_tmp;
-    // the context's buffer, kept from call to call up to kKeepBytes: an
+    // the context's buffer, kept from call to call up to ctx->keep_bytes: an
     // allocation of this size is tens of microseconds, its release some
     // hundreds, and now and then either stalls for tens of milliseconds
     char* buf = nullptr;

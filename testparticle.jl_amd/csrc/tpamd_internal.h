@@ -33,6 +33,7 @@ struct tpamd_ctx {
     // device buffer of the calls that stage or need workspace (ctx_buffer)
     void* d_buf;
     size_t d_buf_bytes;
+    size_t keep_bytes;                      // what of it may stay between calls (ctx_trim)
     unsigned long long* d_steps;
     // pinned host memory of kPinSlots pieces, with one event per piece
     // (stage_in, stage_out), and behind them a word for a step count
@@ -61,8 +62,8 @@ hipError_t adj_bins_seg(const unsigned* keys, const AdjRec<R>* vals, const unsig
 // within one call, which the caller serialises and which ends synchronised.
 // A failure leaves no buffer and no error for the next launch to report.
 hipError_t ctx_buffer(tpamd_ctx* ctx, size_t bytes, void** out);
-// releases it when it has grown past what is kept between calls
-constexpr size_t kKeepBytes = (size_t)4 << 30;
+// Releases it when it has grown past what is kept between calls: 1/16 of the
+// device's memory, as a cell copy may take, or 4 GiB.
 void ctx_trim(tpamd_ctx* ctx);
 
 // Host arrays and the span of the context's device buffer that holds them: a

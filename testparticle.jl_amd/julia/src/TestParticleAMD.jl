@@ -356,7 +356,7 @@ on the uniform ranges x, y, z; `bc` 0 fill NaN, 1 clamp, 2 periodic; `cells`
 adds the cell-replicated device copy), and its gradients with respect to every value
 of A and every initial state (xv0 and targets are 6 x N and 3 x N).  One
 forward pass, which keeps the trajectory in device memory where that takes
-less than 4 GiB and otherwise, or with `checkpoints`, a checkpoint every
+at most 1/16 of what is free, and otherwise, or with `checkpoints`, a checkpoint every
 `ckpt_interval` steps, then a reverse sweep (tpamd_adjoint).  The reference differentiates the same solve with
 ForwardDiff (test/test_derivatives.jl).  `precision = :fp32c` runs the steps
 in float over float storage.  A loss or gradient that is not finite throws

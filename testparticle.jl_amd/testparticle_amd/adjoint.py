@@ -40,8 +40,8 @@ def loss_gradient(prob, *, dt, targets, precision: str = "fp64", ckpt_interval: 
     "fp32c" runs the forward, recompute and reverse steps in float over float
     storage, with the adjoint state scaled by a per-particle power of two.
     The trajectory stays in device memory, a row of 28 (FP32C) or 52 bytes a
-    state, where that takes less than 4 GiB (and half of what is free), which
-    then stay for the next call.  Otherwise, and always with `checkpoints=True`, the forward pass keeps a checkpoint every
+    state, where that takes at most 1/16 of what is free (or 4 GiB), which then
+    stays for the next call.  Otherwise, and always with `checkpoints=True`, the forward pass keeps a checkpoint every
     `ckpt_interval` steps (72 bytes a particle) and the steps between two are
     computed again; dL/d(x0, v0) is the same bit for bit.
     Raises FloatingPointError when the loss or a gradient entry is not finite."""
