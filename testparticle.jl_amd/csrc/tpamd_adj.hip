@@ -321,8 +321,8 @@ constexpr size_t adj_lds_bytes(unsigned nbins)
 // are in flight per thread, each as one group of loads (the row and, by its
 // key, the cell), which hides the gather without occupancy: with SORT the
 // records staged in LDS leave one block of 4 waves a CU.  What is left is
-// memory: a row, a line of cells and a record, 188 B a step in FP32C, run at
-// 5.4 TB/s (131,071 particles x 320 steps, 64^3 float cells: 1.46 ms; with
+// memory: a row, a line of cells and a record, 184 B a step in FP32C, run at
+// 5.3 TB/s (131,071 particles x 320 steps, 64^3 float cells: 1.46 ms; with
 // the trajectory recomputed and the records sorted by a kernel of their own
 // it was 2.9 ms).  512 threads a block, or half the records a block and two
 // blocks a CU, measured within 5 %.

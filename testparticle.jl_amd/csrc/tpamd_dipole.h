@@ -20,8 +20,8 @@
 //     and the arithmetic range;
 //   * the time is carried only where records ask for it.
 // A lane that fails a range test takes the generic arithmetic for that step.
-// Measured: FP64, 262,144 particles x 2,000 steps, 126 -> 99 VALU instructions
-// a step, 2754 -> 1675 us (3.1e11 particle-steps/s); FP32C, 1,000,003 x 1,500,
+// Measured: FP64, 262,144 particles x 2,000 steps, 126 -> 100 VALU instructions
+// a step, 2754 -> 1640-1700 us (3.1e11 particle-steps/s); FP32C, 1,000,003 x 1,500,
 // 122 -> 94, 3347 -> 3172 us (4.7e11; the moves and compares that went issue
 // beside float arithmetic, whose 84 operations are what its time is).
 #pragma once

@@ -9,10 +9,10 @@
 // position for each grid and asked for the second grid's lines only when the
 // first one's were back.  Here the position is located once and both gathers
 // are asked for together.  The arithmetic is the generic policies', so are the
-// results.  Measured, FP64: E and B on 97 x 80 x 113 nodes, 200,001
-// particles x 300 steps: 7.28 -> 2.95 ms (1.56e10 particle-steps/s, 8.0 TB/s
-// of lines); five snapshots of 64 x 61 x 96 nodes, 150,001 x 200: 5.68 ->
-// 2.78 ms.
+// results.  Measured, FP64 with cells: E and B on 97 x 80 x 113 nodes, 200,001
+// particles x 300 steps: 7.28 -> 2.95 ms (1.55e10 particle-steps/s; 4.7 lines a
+// step asked of the L2 and 2.7 missed, 5.2 TB/s); five snapshots of 64 x 61 x
+// 96 nodes, 150,001 x 200: 5.68 -> 2.78 ms (3.5 missed, 4.9 TB/s).
 #pragma once
 
 #include "tpamd_pusher.h"

@@ -820,7 +820,8 @@ struct ChunkSource {
 // are done wait until kRefill are idle: the records and loads are shared by
 // more particles and the long lives get on in between.  They wait kPatience
 // passes at most, as some lanes may hold particles that never leave.  4 M
-// particles of 24 instances, FP32C, median ms: refilled at once 1.22, at 32
+// particles of 24 instances, FP32C, median ms (one set of inputs; the whole batch
+// over others 1.04-1.14 before and 0.91-1.00 now): refilled at once 1.22, at 32
 // idle lanes 1.03, 48 0.99, 56 0.95, 60 0.98; FP64 1.46 -> 1.32; 16 M of 32
 // instances 2.65 -> 2.49; 600,000 with every fifth trapped for 300 steps 1.65,
 // 2.52 without the limit, 1.26 with it.

@@ -14,9 +14,9 @@
 // form below v moves by one component a step and is back after three, and a
 // step takes three permutations.  The position stays in its lane: the
 // component of v that it needs is among the next step's permutations.  In
-// FP64 with E = 0 that is 17 instructions a step instead of 27: 1,024
-// particles x 6,400 steps with every tenth state saved take 418 us instead of
-// 554 (1.57e10 particle-steps/s).
+// FP64 with E = 0 that is 17 vector instructions instead of 27: 1,024
+// particles x 6,400 steps with every tenth state saved take 376 us instead of
+// 526 (1.7e10 particle-steps/s).
 //
 // Every component is formed by the operations of boris_f64 / boris_f32 and
 // their cross products in their order, so the results are those of
