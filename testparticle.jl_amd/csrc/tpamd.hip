@@ -333,11 +333,17 @@ int check_desc(tpamd_ctx* ctx, const tpamd_solve_desc* d, int64_t* nt, int64_t* 
 
 bool is_gridded(const DevField& f) { return f.kind == kFieldGrid || f.kind == kFieldTimeGrid; }
 
-// the field-kind class of a solve: the generic kernels compiled for it
-int solve_class(const KParams& p)
+// the field-kind class of n solves: the generic kernels compiled for it
+int solve_class(const KParams* p, size_t n)
 {
-    const int b = field_class(p.B.kind);
-    return p.e_is_uxb ? b : std::max(b, field_class(p.E.kind));
+    int fk = kFkAnalytic;
+    bool cells = true;                    // in every grid
+    for (size_t i = 0; i < n; ++i)
+        for (const DevField* f : {&p[i].B, p[i].e_is_uxb ? &p[i].B : &p[i].E}) {
+            fk = std::max(fk, field_class(f->kind));
+            cells = cells && (!is_gridded(*f) || f->cells);
+        }
+    return fk == kFkGrid && cells ? (int)kFkCells : fk;
 }
 
 bool same_geometry(const DevField& a, const DevField& b)
@@ -425,6 +431,19 @@ int spec_class(const tpamd_solve_desc* d, const KParams& p, int* emode)
     return ns;
 }
 
+// Whether a solve has the kernels of two gathers a step: gridded E and B on
+// one geometry, or (*time) B a sequence of snapshots; fixed-step Boris, plain
+// records, node arrays that 32-bit offsets reach.
+bool pair_class(const tpamd_solve_desc* d, const KParams& p, bool* time)
+{
+    const bool flat = p.e_is_uxb || p.E.kind == kFieldZero || p.E.kind == kFieldUniform;
+    *time = p.B.kind == kFieldTimeGrid && flat;
+    const bool eb = p.B.kind == kFieldGrid && !p.e_is_uxb && p.E.kind == kFieldGrid && p.E.dtype == p.B.dtype &&
+                    same_geometry(p.E, p.B);
+    return !(d->flags & TPAMD_FLAG_GENERIC_KERNELS) && !d->adaptive && p.alg == TPAMD_ALG_BORIS && p.rec_w == 6 &&
+           (*time || eb) && nodes_bytes(p.B) < 4294967296.0 && (d->precision == TPAMD_FP64 || p.B.dtype == 1);
+}
+
 void select_policy(const tpamd_solve_desc* d, const KParams& p, bool allow_spec, int fk,
                    const LaunchReq& r)
 {
@@ -446,22 +465,17 @@ void select_policy(const tpamd_solve_desc* d, const KParams& p, bool allow_spec,
     // analytic fields have kernels of their own for uniform fields and for
     // the dipole (fixed-step Boris), unless the generic ones are asked for
     const bool special = !(d->flags & TPAMD_FLAG_GENERIC_KERNELS);
-    // two gathers a step: gridded E and B on one geometry (both with cells or
-    // both without), or B a sequence of snapshots (fixed-step Boris, plain
-    // records, node arrays that 32-bit offsets reach).  Float nodes at FP32C
-    // are the exception: with a wave on every SIMD the generic kernels are the
-    // faster ones (100,000 particles, E and B of 28^3 1.4 times, of 80^3 1.15;
-    // 200,000, snapshots of 56^3 1.09), for E and B beyond 4 MiB of L2 always
-    // (500 particles, 80^3: 1.05); elsewhere the pair is (50,000 particles,
-    // snapshots of 28^3: 1.7 times)
-    const bool flat = p.e_is_uxb || p.E.kind == kFieldZero || p.E.kind == kFieldUniform;
-    const bool time = p.B.kind == kFieldTimeGrid && flat;
-    const bool eb = p.B.kind == kFieldGrid && !p.e_is_uxb && p.E.kind == kFieldGrid && p.E.dtype == p.B.dtype &&
-                    (p.E.cells != nullptr) == (p.B.cells != nullptr) && same_geometry(p.E, p.B);
+    // two gathers a step, both grids with cells or both without.  Float nodes
+    // at FP32C are the exception: with a wave on every SIMD the generic kernels
+    // are the faster ones (100,000 particles, E and B of 28^3 1.4 times, of 80^3
+    // 1.15; 200,000, snapshots of 56^3 1.09), for E and B beyond 4 MiB of L2
+    // always (500 particles, 80^3: 1.05); elsewhere the pair is (50,000
+    // particles, snapshots of 28^3: 1.7 times)
+    bool time = false;
+    const bool pair = !r.batch && pair_class(d, p, &time);
     const bool nodes32 = d->precision == TPAMD_FP32C && !p.B.cells &&
-                         (p.N >= 65536 || (eb && 2.0 * nodes_bytes(p.B) > 4.0 * 1048576.0));
-    if (special && !r.batch && !r.adaptive && p.alg == TPAMD_ALG_BORIS && p.rec_w == 6 && (time || eb) && !nodes32 &&
-        nodes_bytes(p.B) < 4294967296.0 && (d->precision == TPAMD_FP64 || p.B.dtype == 1)) {
+                         (p.N >= 65536 || (!time && 2.0 * nodes_bytes(p.B) > 4.0 * 1048576.0));
+    if (pair && !nodes32 && (time || (p.E.cells != nullptr) == (p.B.cells != nullptr))) {
         const bool per = p.B.extrap == kExtrapPeriodic, cells = p.B.cells != nullptr;
         if (d->precision == TPAMD_FP32C) launch_pair32(r, time, p.e_is_uxb != 0, per, cells);
         else launch_pair64(r, time, p.e_is_uxb != 0, per, p.B.dtype == 1, cells);
@@ -469,10 +483,12 @@ void select_policy(const tpamd_solve_desc* d, const KParams& p, bool allow_spec,
     }
     if (d->precision == TPAMD_FP64) {
         if (fk == kFkMesh) launch_generic64_mesh(r, p.alg);
+        else if (fk == kFkCells) launch_generic64_cells(r, p.alg);
         else if (fk == kFkGrid) launch_generic64(r, p.alg);
         else launch_generic64_analytic(r, p.alg, special);
     } else {
         if (fk == kFkMesh) launch_generic32_mesh(r, p.alg);
+        else if (fk == kFkCells) launch_generic32_cells(r, p.alg);
         else if (fk == kFkGrid) launch_generic32(r, p.alg);
         else launch_generic32_analytic(r, p.alg, special);
     }
@@ -544,21 +560,31 @@ int build_cells(tpamd_ctx* ctx, tpamd_field* f, hipStream_t st, bool asked)
 //     cells fit as well (up to 0.5 MiB of nodes), double ones are 1.2-1.45 times
 //     faster at any number (16^3, 500 particles: 2.53 -> 2.11 ns), float ones
 //     0.88-1.0.
+//   * The generic kernels (records with fields, other multistep orders): double
+//     ones 1.05-1.2 times faster within the L2 at any number and 1.1-2.1 beyond
+//     (64^3, 500 particles 1.1-1.5 ns, 100,000 0.015-0.04); float ones 0.88-1.08
+//     within and 1.05-2.2 beyond (96^3, 500 particles 0.7-1.0, 100,000 0.01-0.023).
 //   * The gradient, whose reverse sweep reads a cell's 24 values as they lie:
 //     never slower within it, 1.1-1.46 times for double (48^3, 5,000 particles),
 //     1.0-1.2 for float; beyond it as above.
-double cells_gain(const DevField& B, const DevField* E, long long N, bool gradient)
+enum class CellUse { special, generic, gradient };
+double cells_gain(const DevField& B, const DevField* E, long long count, CellUse use)
 {
+    const double N = (double)std::max(count, 1LL);
     auto lone = [](const DevField& f) { return is_gridded(f) ? nodes_bytes(f) * (f.nsnap > 1 ? 2.0 : 1.0) : 0.0; };
     const bool both = E && is_gridded(B);
     const DevField& f = is_gridded(B) ? B : *E;
     const double mib = (lone(B) + (E ? lone(*E) : 0.0)) / 1048576.0;
-    if (mib > 4.0)
-        return std::max(mib > 16.0 ? 0.045 : 0.028, (f.dtype == 1 ? 1000.0 : 1800.0) / (double)std::max(N, 1LL));
-    if (gradient) return f.dtype == 1 ? 0.002 : std::max(0.006, 360.0 / (double)N);
-    if (f.dtype != 1 && mib <= 0.5) return std::max(N >= 65536 ? 0.015 : 0.004, 200.0 / (double)std::max(N, 1LL));
-    if (both) return f.dtype == 1 ? 0.015 : 0.0;
-    return N >= (f.nsnap > 1 && f.dtype != 1 ? 131072 : 65536) ? 0.018 : 0.0;
+    const bool f32 = f.dtype == 1;
+    if (use == CellUse::generic) {
+        if (mib > 4.0) return std::max(mib > 16.0 ? (f32 ? 0.03 : 0.04) : (f32 ? 0.012 : 0.015), (f32 ? 300.0 : 600.0) / N);
+        return f32 ? 0.0 : std::max(0.004, 250.0 / N);
+    }
+    if (mib > 4.0) return std::max(mib > 16.0 ? 0.045 : 0.028, (f32 ? 1000.0 : 1800.0) / N);
+    if (use == CellUse::gradient) return f32 ? 0.002 : std::max(0.006, 360.0 / N);
+    if (!f32 && mib <= 0.5) return std::max(N >= 65536.0 ? 0.015 : 0.004, 200.0 / N);
+    if (both) return f32 ? 0.015 : 0.0;
+    return N >= (f.nsnap > 1 && !f32 ? 131072.0 : 65536.0) ? 0.018 : 0.0;
 }
 
 // A solve of `gathers` field evaluations from a field's node array builds the
@@ -598,13 +624,13 @@ void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, double g
 
 // The fields of a solve of N particles and `gathers` evaluations as its
 // kernels see them: with cells where that is faster, or where the caller asked
-// for a copy.  (The results are the same bits.)
+// for a copy and has kernels made for it.  (The results are the same bits.)
 void settle_cells(tpamd_ctx* ctx, const tpamd_field* E, const tpamd_field* B, long long N, double gathers,
-                  hipStream_t st, KParams& p, bool gradient = false)
+                  CellUse use, hipStream_t st, KParams& p)
 {
     const bool e = !p.e_is_uxb && is_gridded(E->d);
     if (!e && !is_gridded(B->d)) return;
-    const double gain = cells_gain(B->d, e ? &E->d : nullptr, N, gradient);
+    const double gain = cells_gain(B->d, e ? &E->d : nullptr, N, use);
     if (gain > 0.0) {
         offer_cells(ctx, B, gathers, gain, st);
         if (e) offer_cells(ctx, E, gathers, gain, st);
@@ -612,7 +638,7 @@ void settle_cells(tpamd_ctx* ctx, const tpamd_field* E, const tpamd_field* B, lo
     p.B = B->d;
     p.E = E->d;
     const bool asked = (B->d.cells && !B->cells_auto) || (e && E->d.cells && !E->cells_auto);
-    if (gain <= 0.0 && !asked) p.B.cells = p.E.cells = nullptr;
+    if (gain <= 0.0 && (!asked || use == CellUse::generic)) p.B.cells = p.E.cells = nullptr;
 }
 
 // Validates the descriptor and fills the kernel parameter block (everything
@@ -761,7 +787,11 @@ int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fiel
     p.span = (int)(64 * ppl);
     if (!(desc->flags & TPAMD_FLAG_GENERIC_KERNELS)) {
         // an adaptive particle's steps are not known: two evaluations at least
-        settle_cells(ctx, E, B, N, (double)N * (desc->adaptive ? 2.0 : (double)nt + 1.0), st, p);
+        int emode;
+        bool time;
+        const bool special = spec_class(desc, p, &emode) >= 0 || pair_class(desc, p, &time);
+        settle_cells(ctx, E, B, N, (double)N * (desc->adaptive ? 2.0 : (double)nt + 1.0),
+                     special ? CellUse::special : CellUse::generic, st, p);
     }
     if (N > 0) {
         const long long threads = desc->adaptive ? (N + p.span - 1) / p.span * 64 : N;
@@ -774,7 +804,7 @@ int solve_enqueue(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_fiel
         r.b = block;
         r.st = st;
         r.p = &p;
-        select_policy(desc, p, true, solve_class(p), r);
+        select_policy(desc, p, true, solve_class(&p, 1), r);
         HIP_TRY(ctx, hipGetLastError());
         HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
     }
@@ -851,10 +881,9 @@ int batch_table(tpamd_batch* b, const tpamd_field* const* E, const tpamd_field* 
     int em0 = 0;
     const int ns0 = spec_class(desc, p0, &em0);
     b->allow_spec = ns0 >= 0;
-    b->fk = kFkAnalytic;
+    b->fk = solve_class(b->table.data(), b->table.size());
     for (const KParams& p : b->table) {
         int em = 0;
-        b->fk = std::max(b->fk, solve_class(p));
         b->allow_spec = b->allow_spec && spec_class(desc, p, &em) == ns0 && em == em0 && p.B.dtype == p0.B.dtype &&
                         (p.B.extrap == kExtrapPeriodic) == (p0.B.extrap == kExtrapPeriodic) &&
                         (p.B.cells != nullptr) == (p0.B.cells != nullptr);
@@ -1664,7 +1693,7 @@ int32_t tpamd_adjoint(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpamd_
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     Drain drain{ctx->stream};                       // adjoint_launch leaves early where it fails
     // forward and reverse; the FP64 kernels on float nodes read no cells
-    if (bf32 == f32) settle_cells(ctx, &zero, B, N, 2.0 * (double)N * (double)nt, ctx->stream, p, true);
+    if (bf32 == f32) settle_cells(ctx, &zero, B, N, 2.0 * (double)N * (double)nt, CellUse::gradient, ctx->stream, p);
     else p.B.cells = nullptr;
     auto launch = [&](bool ckpt) {
         const bool cells = p.B.cells != nullptr;    // gathers from the cell-replicated copy
@@ -1732,7 +1761,7 @@ int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpa
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     char* b = nullptr;
     HIP_TRY(ctx, call_buffer(ctx, need, (void**)&b));
-    settle_cells(ctx, E, B, N, 0.0, ctx->stream, p);     // builds none
+    settle_cells(ctx, E, B, N, 0.0, CellUse::generic, ctx->stream, p);     // builds none
     FoArgs a;
     a.state = (double*)b; b += al(b_st);
     a.iters = (long long*)b; b += al(b_it);
@@ -1757,7 +1786,7 @@ int32_t tpamd_fo_segment(tpamd_ctx* ctx, const tpamd_solve_desc* desc, const tpa
         HIP_TRY(ctx, hipMemcpyAsync(a.iters, iters, b_it, hipMemcpyHostToDevice, st));
         HIP_TRY(ctx, hipMemcpyAsync(a.flags, flags, b_i, hipMemcpyHostToDevice, st));
         HIP_TRY(ctx, hipEventRecord(ctx->ev0, st));
-        launch_fo_segment(p, a, solve_class(p), st);
+        launch_fo_segment(p, a, solve_class(&p, 1), st);
         HIP_TRY(ctx, hipGetLastError());
         HIP_TRY(ctx, hipEventRecord(ctx->ev1, st));
         HIP_TRY(ctx, hipMemcpyAsync(state, a.state, b_st, hipMemcpyDeviceToHost, st));

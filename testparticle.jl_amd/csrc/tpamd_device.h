@@ -437,11 +437,11 @@ __device__ __forceinline__ void node3_f64(const DevField& f, long long idx, doub
 }
 
 // build_interpolator(CartesianGrid, A::4D, ...) + linear_interp,
-// src/utility/interpolation.jl:119-148, :203-206, :217-235; from the cells
-// where the field has them (same values, same blend order)
+// src/utility/interpolation.jl:119-148, :203-206, :217-235; CELLS: from the
+// cell-replicated copy (same values, same blend order)
+template <bool CELLS>
 __device__ __forceinline__ void grid_f64(const DevField& f, const double x[3], double out[3], int snap = 0)
 {
-    const void* base = snapshot(f, snap);
     int i0[3], i1[3];
     double w[3];
 #pragma unroll
@@ -477,12 +477,13 @@ __device__ __forceinline__ void grid_f64(const DevField& f, const double x[3], d
             i1[d] = i0[d] + 1;
         }
     }
-    if (f.cells) {
+    if constexpr (CELLS) {
         const void* cells = snapshot_cells(f, snap);
         if (f.dtype == 1) trilinear_cell<float, double>(cells, cell_offset(f, i0), w, out);
         else trilinear_cell<double, double>(cells, cell_offset(f, i0), w, out);
         return;
     }
+    const void* base = snapshot(f, snap);
     const long long nx = f.n[0], nxy = (long long)f.n[0] * f.n[1];
     double a[3], b[3], c00[3], c10[3], c01[3], c11[3];
     node3_f64(f, base, i0[0] + nx * i0[1] + nxy * i0[2], a);
@@ -526,8 +527,9 @@ __device__ __forceinline__ int time_bracket(const DevField& f, double t, double&
 // (zero, uniform, affine, dipole), + uniform grids and their time sequences,
 // + meshes (through the out-of-line mesh evaluator).  A solve takes the
 // smallest class that holds its E and B, so kernels never carry the code
-// (and the registers) of field kinds they cannot meet.
-enum { kFkAnalytic = 0, kFkGrid = 1, kFkMesh = 2 };
+// (and the registers) of field kinds they cannot meet.  kFkCells is kFkGrid
+// with every grid read from its cell-replicated copy; the others read nodes.
+enum { kFkAnalytic = 0, kFkGrid = 1, kFkMesh = 2, kFkCells = 3 };
 
 __host__ __device__ inline int field_class(int kind)
 {
@@ -576,7 +578,7 @@ __device__ __forceinline__ void field_f64(const DevField& f, const double x[3], 
         return;
     case kFieldGrid:
         if constexpr (FK >= kFkGrid) {
-            grid_f64(f, x, o);
+            grid_f64<FK == kFkCells>(f, x, o);
             return;
         }
         break;
@@ -585,12 +587,12 @@ __device__ __forceinline__ void field_f64(const DevField& f, const double x[3], 
             double w;
             const int k = time_bracket(f, t, w);
             if (k == 0 || k >= f.nsnap) {
-                grid_f64(f, x, o, k == 0 ? 0 : f.nsnap - 1);
+                grid_f64<FK == kFkCells>(f, x, o, k == 0 ? 0 : f.nsnap - 1);
                 return;
             }
             double a[3], b[3];
-            grid_f64(f, x, a, k - 1);
-            grid_f64(f, x, b, k);
+            grid_f64<FK == kFkCells>(f, x, a, k - 1);
+            grid_f64<FK == kFkCells>(f, x, b, k);
 #pragma unroll
             for (int c = 0; c < 3; ++c) o[c] = (1.0 - w) * a[c] + w * b[c];   // interpolation.jl:377
             return;
@@ -741,8 +743,8 @@ __device__ __forceinline__ void field_jac_f64(const DevField& f, const double x[
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 3; ++j) J[i][j] = (1.0 - w) * J1[i][j] + w * J2[i][j];
-        grid_f64(f, x, a, k - 1);
-        grid_f64(f, x, b, k);
+        grid_f64<FK == kFkCells>(f, x, a, k - 1);
+        grid_f64<FK == kFkCells>(f, x, b, k);
         const double dtk = f.times[k] - f.times[k - 1];
 #pragma unroll
         for (int i = 0; i < 3; ++i) dBdt[i] = (b[i] - a[i]) / dtk;
@@ -966,7 +968,7 @@ __device__ __forceinline__ void node3_f32(const T* __restrict__ d, long long idx
 
 // Trilinear gather in float from frame-relative coordinates (frame origin =
 // the grid origin, so s = (hi + lo) / h without cancellation).
-template <typename T>
+template <typename T, bool CELLS>
 __device__ __forceinline__ void grid_f32_t(const DevField& f, const Pos32& x, float out[3], int snap = 0)
 {
     int i0[3], i1[3];
@@ -1003,7 +1005,7 @@ __device__ __forceinline__ void grid_f32_t(const DevField& f, const Pos32& x, fl
             i1[d] = i0[d] + 1;
         }
     }
-    if (f.cells) {
+    if constexpr (CELLS) {
         trilinear_cell<T, float>(snapshot_cells(f, snap), cell_offset(f, i0), w, out);
         return;
     }
@@ -1110,8 +1112,8 @@ __device__ __forceinline__ void field_f32(const KParams& p, const DevField& f, c
         return;
     case kFieldGrid:
         if constexpr (FK >= kFkGrid) {
-            if (f.dtype == 1) grid_f32_t<float>(f, x, o);
-            else grid_f32_t<double>(f, x, o);
+            if (f.dtype == 1) grid_f32_t<float, FK == kFkCells>(f, x, o);
+            else grid_f32_t<double, FK == kFkCells>(f, x, o);
         } else {
             o[0] = o[1] = o[2] = 0.0f;
         }
@@ -1126,11 +1128,11 @@ __device__ __forceinline__ void field_f32(const KParams& p, const DevField& f, c
         const int k0 = k == 0 ? 0 : k - 1, k1 = k >= f.nsnap ? f.nsnap - 1 : k;
         float a[3], b[3];
         if (f.dtype == 1) {
-            grid_f32_t<float>(f, x, a, k0);
-            if (k1 != k0) grid_f32_t<float>(f, x, b, k1);
+            grid_f32_t<float, FK == kFkCells>(f, x, a, k0);
+            if (k1 != k0) grid_f32_t<float, FK == kFkCells>(f, x, b, k1);
         } else {
-            grid_f32_t<double>(f, x, a, k0);
-            if (k1 != k0) grid_f32_t<double>(f, x, b, k1);
+            grid_f32_t<double, FK == kFkCells>(f, x, a, k0);
+            if (k1 != k0) grid_f32_t<double, FK == kFkCells>(f, x, b, k1);
         }
         if (k == 0 || k >= f.nsnap) {
             o[0] = a[0]; o[1] = a[1]; o[2] = a[2];

@@ -102,6 +102,7 @@ void launch_fo_segment(const KParams& p, const FoArgs& a, int fk, hipStream_t st
 {
     const dim3 block(256), grid((unsigned)((p.N + 255) / 256));
     if (fk == kFkMesh) hipLaunchKernelGGL((k_fo_segment<S64M>), grid, block, 0, st, p, a);
+    else if (fk == kFkCells) hipLaunchKernelGGL((k_fo_segment<S64C>), grid, block, 0, st, p, a);
     else if (fk == kFkGrid) hipLaunchKernelGGL((k_fo_segment<S64>), grid, block, 0, st, p, a);
     else hipLaunchKernelGGL((k_fo_segment<S64A>), grid, block, 0, st, p, a);
 }

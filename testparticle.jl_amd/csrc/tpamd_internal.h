@@ -140,12 +140,14 @@ struct LaunchReq {
 };
 
 // generic kernels, FP64 and FP32C, per field-kind class: analytic fields
-// (tpamd_gen64a/32a.hip), + grids (tpamd_gen64/32.hip), + meshes
-// (tpamd_gen64m/32m.hip)
+// (tpamd_gen64a/32a.hip), + grids (nodes tpamd_gen64/32.hip, cells
+// tpamd_gen64c/32c.hip), + meshes (tpamd_gen64m/32m.hip)
 void launch_generic64_analytic(const LaunchReq& r, int alg, bool special);
 void launch_generic32_analytic(const LaunchReq& r, int alg, bool special);
 void launch_generic64(const LaunchReq& r, int alg);
 void launch_generic32(const LaunchReq& r, int alg);
+void launch_generic64_cells(const LaunchReq& r, int alg);
+void launch_generic32_cells(const LaunchReq& r, int alg);
 void launch_generic64_mesh(const LaunchReq& r, int alg);
 void launch_generic32_mesh(const LaunchReq& r, int alg);
 // specialised gridded-B kernels (tpamd_spec64/32.hip): emode kEUniform /

@@ -196,9 +196,11 @@ struct S32CT {
 // generic policies per field-kind class: analytic fields, + grids, + meshes
 using S64A = S64T<kFkAnalytic>;
 using S64 = S64T<kFkGrid>;
+using S64C = S64T<kFkCells>;
 using S64M = S64T<kFkMesh>;
 using S32CA = S32CT<kFkAnalytic>;
 using S32C = S32CT<kFkGrid>;
+using S32CC = S32CT<kFkCells>;
 using S32CM = S32CT<kFkMesh>;
 
 // a policy whose fixed-step Boris kernel forms the update's rotation vectors

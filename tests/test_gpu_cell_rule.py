@@ -92,3 +92,44 @@ def taken(kind, m, dtype, n, nt):
 ])
 def test_when_a_copy_is_built(case, built):
     assert (taken(*case) > 8 << 20) == built
+
+
+# solves that only the generic kernels cover: their kernels for cells and for
+# nodes, singly and in batches, on small grids and beyond the L2
+@pytest.mark.parametrize("bc", list(BCS))
+@pytest.mark.parametrize("precision,dtype", [("fp64", np.float64), ("fp64", np.float32), ("fp32c", np.float32)])
+@pytest.mark.parametrize("kind", ["one", "pair", "time"])
+@pytest.mark.parametrize("shape,n", [((9, 7, 11), 65), ((9, 7, 11), 20001), ((66, 60, 64), 9001)])
+@pytest.mark.parametrize("alg,kw", [(TP.Boris(), dict(dt=0.3, savestepinterval=9, save_fields=True)),
+                                    (TP.MultistepBoris(6, n=3), dict(dt=0.3, save_everystep=False)),
+                                    (TP.AdaptiveBoris(0.1), dict(max_steps=20, save_everystep=False, save_fields=True))])
+def test_generic_kernels_on_either_layout(kind, precision, dtype, bc, shape, n, alg, kw):
+    xv = particles(n)
+    kw = dict(kw, precision=precision, isoutside=None if bc == "periodic" else TP.OutsideGrid())
+
+    def prob(layout):
+        E, B = fields(kind, shape, bc, dtype, layout)
+        return TP.TraceProblem(xv, (0.0, 27 * 0.3), (Q2M, TP.mi, E, B, TP.ZeroField()))
+
+    def bits(s):
+        w = np.arange(s.u_all.shape[1]) < s.lengths[:, None]
+        return s.lengths, s.retcodes, s.u_all[w].view(np.int64), s.t_all[w].view(np.int64)
+
+    p = {layout: prob(layout) for layout in ("nodes_only", "nodes", "cells")}
+    want = bits(TP.solve(p["nodes_only"], alg, **kw))
+    got = [bits(TP.solve(p[layout], alg, **kw)) for layout in ("nodes", "nodes", "cells")]
+    got += [bits(s) for layout in ("nodes", "cells") for s in TP.solve_batch([p[layout]] * 2, alg, **kw)]
+    got += [bits(s) for s in TP.solve_batch([p["cells"], p["nodes"]], alg, **kw)]
+    for g in got:
+        for a, b in zip(g, want):
+            np.testing.assert_array_equal(a, b)
+
+
+def test_full_orbit_segments_on_cells():
+    from test_gpu_hybrid import _lockstep
+    B = grid((20, 17, 23), 3, "periodic", np.float64, "cells", scale=1e-9)
+    xv = particles(97)
+    q2m = TP.qi / TP.mi
+    Tg = 2 * np.pi / (q2m * 5e-9)
+    prob = TP.TraceHybridProblem(xv, (0.0, 8 * Tg), (q2m, TP.mi, TP.UxBField([2e5, 0.0, 1e5], B), B, TP.ZeroField()))
+    _lockstep(prob, TP.hybrid(dtmax=Tg / 20, dtmin=Tg / 400, check_interval=40), xv, K=7)
