@@ -588,15 +588,20 @@ double cells_gain(const DevField& B, const DevField* E, long long count, CellUse
 }
 
 // A solve of `gathers` field evaluations from a field's node array builds the
-// cell-replicated copy first, on its stream, where that repays itself within
-// the solve, and the field keeps it.  Building takes some 50 us and 0.45 us a
-// MB of cells, and 120 us more to allocate above 64 MB (6 MB 49 us, 50 MB 62,
-// 113 MB 200-275, 170 MB 195-260, 403 MB 280-330, 1.36 GB 720-850; the
-// first of a size in a process up to 0.5 ms).  The gathers are those of a solve
-// whose particles all live to its end: lives that a boundary ends in the first
-// steps build a copy for nothing, once a field (100,000 particles gone within
-// two of 1,000 steps, 128^3: 0.20 -> 0.6 ms).  A copy takes at most 1/16 of the
-// free memory, and a caller that dropped a field's copy gets none.  The copy
+// cell-replicated copy first, on its stream, once the field's solves to the
+// end of this one have had as much to save as building takes, and the field
+// keeps it: a first solve builds it where it repays itself within the solve,
+// repeated smaller ones after a few, having lost by then what building takes
+// (8 snapshots of 83 x 81 x 89, FP32C, 65,317 particles x 111 steps: 0.44 ms,
+// from the second on 0.27; 130^3 double, 71,049 x 57, 2 substeps: 0.59, 0.30).
+// Building takes some 50 us and 0.45 us a MB of cells, and 120 us more to
+// allocate above 64 MB (6 MB 49 us, 50 MB 62, 113 MB 200-275, 170 MB 195-260,
+// 403 MB 280-330, 1.36 GB 720-850; the first of a size in a process up to
+// 0.5 ms).  The gathers are those of a solve whose particles all live to its
+// end: lives that a boundary ends in the first steps build a copy for nothing,
+// once a field (100,000 particles gone within two of 1,000 steps, 128^3:
+// 0.20 -> 0.6 ms).  A copy takes at most 1/16 of the free memory, and a caller
+// that dropped a field's copy gets none.  The copy
 // counts as built at once: the caller has checked its arguments, and leaves,
 // also with an error, only when the stream has been waited for (Drain), so
 // that the next solve finds it on any stream.
@@ -607,8 +612,9 @@ void offer_cells(tpamd_ctx* ctx, const tpamd_field* cf, double gathers, double g
     const bool time = f->d.kind == kFieldTimeGrid;
     const double one = cells_bytes(f->d), all = one * (time ? f->d.nsnap : 1);
     if (f->d.nsnap > 1) gathers *= 2.0;                           // blends two snapshots
-    if (one >= 4294967296.0 || gathers * gain < 5.0e4 + 4.5e-4 * all + (all > 6.4e7 ? 1.2e5 : 0.0))
-        return;
+    f->cells_owed += gathers * gain;
+    if (one >= 4294967296.0 || f->cells_owed < 5.0e4 + 4.5e-4 * all + (all > 6.4e7 ? 1.2e5 : 0.0)) return;
+    f->cells_owed = 0.0;                 // built or not: the memory is not asked for at each solve
     size_t mem_free = 0, mem_total = 0;
     if (hipMemGetInfo(&mem_free, &mem_total) != hipSuccess || all > (double)mem_free / 16.0) {
         (void)hipGetLastError();
@@ -1103,6 +1109,7 @@ static int32_t new_field(tpamd_ctx* ctx, tpamd_field** out, int kind)
     f->cells_data = nullptr;
     f->cells_off = false;
     f->cells_auto = false;
+    f->cells_owed = 0.0;
     f->owner = ctx;
     f->src = nullptr;
     f->bytes = 0;

@@ -19,6 +19,7 @@ struct tpamd_field {
     bool cells_off;          // the caller dropped the copy: no solve builds it again
     bool cells_auto;         // a solve built it and the caller has not asked for it: no batch uses it,
                              // and it may go between calls (relieve)
+    double cells_owed;       // ns that solves since the last offer would have saved on a copy (offer_cells)
     tpamd_ctx* owner;        // the context whose calls use the field
     const tpamd_field* src;  // UxB: the B field it was built from
     size_t bytes;
